@@ -920,6 +920,10 @@ HXA_DEV void gemm_body(const GemmParams &p, const int bid, const int z) {
     mfma_range(ca[0], cb[0], 0, 2);
     __builtin_amdgcn_sched_barrier(0);
     wait_stage<BM, BN, FMT, ASYM, NW, NS - 2>(wave);  // tile kt+1 complete; tiles kt+2 .. kt+NS-1 may still fly
+    // lgkmcnt(0): this wave's fragment reads of stage kt are in registers. Its first MFMAs only waited for the ones they
+    // use, and past the barrier other waves load into that stage: a line that hits in L1 can land before a read that is
+    // still queued behind another workgroup's on the same CU
+    __builtin_amdgcn_s_waitcnt(0xc07f);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();             // stage kt+1 visible; every wave holds its stage kt fragments
     asm volatile("" ::: "memory");
