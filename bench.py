@@ -308,8 +308,7 @@ FAMILIES = {  # family -> the stages whose launches it is
 
 
 def _kname(pk):
-    return (f"{'gemm_pp_kernel' if pk['waves'] == 9 else 'gemm_kernel'} {pk['bm']}x{pk['bn']}"
-            f" ({8 if pk['waves'] == 9 else pk['waves']} waves)")
+    return f"gemm_kernel {pk['bm']}x{pk['bn']} ({8 if pk['bm'] * pk['bn'] > 128 * 128 else 4} waves)"
 
 
 def family_launchers(L, hip, s):

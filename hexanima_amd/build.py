@@ -19,7 +19,8 @@ LIB = os.path.join(HERE, "libhexanima_hip.so")
 MOSS_LIB = os.path.join(HERE, "libhexanima_moss.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 PROGRAMS = ["hxa_run", "hxa_blk"]
-SOURCES = ["gemm.hip", "attention.hip", "elementwise.hip", "runtime.hip", "dit.hip", "noalloc.hip"]
+SOURCES = ["gemm.hip", "gemm_f16.hip", "gemm_q8.hip", "gemm_q4.hip",
+           "attention.hip", "elementwise.hip", "runtime.hip", "dit.hip", "noalloc.hip"]
 
 ARCH = os.environ.get("HXA_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")

@@ -23,17 +23,17 @@ struct HxaGemm {
   long ldo_t;
   int split_col;
   int force_bm, force_bn;  // 0 = automatic tile choice
-  int force_nw;            // waves per workgroup with a forced tile: 0 / 4, 8, or 9 (the ping-pong kernel)
+  int force_nw;            // a forced tile's wave count name: 0 / 4, 8 or 9 (tile_built)
   // STORE with head norm: columns [0, hn_cols) (multiple of 128) get per-head RMSNorm * gain (gain hn_g0 for columns
   // < hn_gsplit, hn_g1 above) and, with hn_cos / hn_sin [hn_ttab][64], RoPE at token m % hn_ttab (kern.c:163-197)
   int hn_cols, hn_gsplit, hn_ttab;
   const float *hn_g0, *hn_g1, *hn_cos, *hn_sin;
-  // a GEMV to run with this GEMM: in workgroups appended to a one-slice ping-pong grid whose last round leaves at
+  // a GEMV to run with this GEMM: in workgroups appended to a one-slice 8-wave grid whose last round leaves at
   // least 16 CUs idle, else as its own launch after the GEMM (nullptr: none)
   const HxaSideGemv *side;
 };
 int hxa_gemm_launch(const HxaGemm &g, hipStream_t st);
-// the tile hxa_gemm_launch would run g on (bm x bn, nw waves per workgroup, 9 = the ping-pong kernel) and the
+// the tile hxa_gemm_launch would run g on (bm x bn under the name nw) and the
 // rounds of workgroups over the CUs it would take (tile grid x ksplit / CUs, rounded up); HXA_OK, or the error
 // hxa_gemm_launch would return
 int hxa_gemm_plan(const HxaGemm &g, int *bm, int *bn, int *nw, int *rounds);
@@ -58,7 +58,7 @@ bool hxa_gemm_xattn_fits(int M, int N);
 // whether hxa_gemm_pair_launch(g0, g1) would be one launch that takes no more rounds of workgroups over the CUs than
 // g0 alone (g1 only fills CUs g0 leaves idle)
 bool hxa_gemm_pair_fits(const HxaGemm &g0, const HxaGemm &g1);
-// G GEMMs of one shape and weight format (ksplit 1, no prefetch) in one launch on the ping-pong 192x256 tile, each
+// G GEMMs of one shape and weight format (ksplit 1, no prefetch) in one launch on the 192x256 tile, each
 // with its own operands and epilogue. prepare fills params_host (hxa_gemm_group_param_bytes(G) bytes, to be copied
 // to device memory as they are) and returns the tiles per GEMM and the launch format; the device copy stays valid
 // while the GEMMs' operands stay where they are.

@@ -500,7 +500,7 @@ constexpr long DQ_MIN_ROWS = 1024;
 // from this many rows on the pass also pays for the wide projections (qkv, MLP up / up-gate)
 constexpr long DQ_WIDE_ROWS = 4096;
 // int8 / int4 attention-output and MLP-down projections at DQ_MIN_ROWS .. DQ_WIDE_ROWS rows (no LoRA) run fused,
-// split-K 4 on the ping-pong tiles, into four fp16 partials that the next norm adds: those tiles hide the
+// split-K 4 on the 8-wave tiles, into four fp16 partials that the next norm adds: those tiles hide the
 // dequantisation under their MFMAs, and no fp16 copy of the weight goes through memory (1536 tokens, 2.9B-class
 // MLP-down 10240 -> 2560: 80 us fused against 15.5 us of dequantisation + 84.5 us of fp16 GEMM in the step).
 // Not with the reference's rounding points (round_ref: mega_block), which round o once and the MLP-down in two halves.

@@ -167,7 +167,7 @@ def device_info():
 
 
 def gemm_pick(M, N, K, fmt, ksplit=1, epi=0, norm_cols=0):
-    """the tile hxa_gemm chooses: {'bm', 'bn', 'waves' (9 = ping-pong kernel), 'rounds'}"""
+    """the tile hxa_gemm chooses: {'bm', 'bn', 'waves' (its name for gemm_tile), 'rounds'}"""
     init()
     bm, bn, w, r = I(), I(), I(), I()
     check(lib().hxa_gemm_pick(M, N, K, fmt, ksplit, epi, norm_cols, C.byref(bm), C.byref(bn), C.byref(w), C.byref(r)),

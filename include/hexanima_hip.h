@@ -149,9 +149,10 @@ int hxa_clock_record(int kind, void *rec, long nrec);
 int hxa_gemm(const void *A, long lda, int M, int fmt, const void *w, const void *s, const void *z, int N, int K,
              int ksplit, int epi, void *out, long ldo, long out_zstride, float *x, long ldx, const float *gate,
              void *out_t, long ldo_t, int split_col, void *stream);
-/* same, with an explicit tile shape (tests / tuning). waves per workgroup 4 (0 = 4): bm x bn in {192x256, 192x192,
- * 192x128, 256x128, 128x256, 128x128, 64x128, 128x64}; 8: {192x256, 192x128, 128x256, 128x128}; 9, the ping-pong
- * kernel: {256x256, 192x256, 128x256, 128x128 (not int4)}. int4 weights need bn >= 128, SiTU bn % 128 == 0. */
+/* same, with an explicit tile shape (tests / tuning). Each tile has one kernel per weight format (8 waves above 128x128,
+ * 4 or 8 at and below it), under every name that waves gives it: 4 (0 = 4): bm x bn in {192x256, 192x192, 192x128,
+ * 256x128, 128x256, 128x128, 64x128, 64x64, 128x64 (not int4)}; 8: {192x256, 192x128, 128x256, 128x128}; 9: {256x256,
+ * 192x256, 128x256, 256x192} and, not int4, {256x128, 192x128, 128x128}. SiTU and head norms need bn % 128 == 0. */
 int hxa_gemm_tile(const void *A, long lda, int M, int fmt, const void *w, const void *s, const void *z, int N, int K,
                   int ksplit, int epi, void *out, long ldo, long out_zstride, float *x, long ldx, const float *gate,
                   int bm, int bn, int waves, void *stream);
@@ -171,8 +172,8 @@ long hxa_linear_ws_bytes(int M, int N, int K, int fmt);
 int hxa_sum_partials(const float *p, int nslice, long zstride, long ldp, int M, int N, void *out, long ldo,
                      void *stream);
 /* The tile hxa_gemm chooses for these sizes, weight format (HXA_W_*, KTILED ignored), split and epilogue
- * (norm_cols > 0: hxa_gemm_headnorm's head-normed columns): *bm x *bn with *waves per workgroup (9: the ping-pong
- * kernel) and *rounds of workgroups over the GPU's CUs. Returns 0, or the error hxa_gemm would return for these
+ * (norm_cols > 0: hxa_gemm_headnorm's head-normed columns): *bm x *bn with *waves, the name hxa_gemm_tile takes
+ * it under, and *rounds of workgroups over the GPU's CUs. Returns 0, or the error hxa_gemm would return for these
  * sizes. No counterpart in the reference (its GEMM has one tile); for tuning and benchmarks. */
 int hxa_gemm_pick(int M, int N, int K, int fmt, int ksplit, int epi, int norm_cols, int *bm, int *bn, int *waves,
                   int *rounds);

@@ -1,0 +1,91 @@
+"""The GEMM kernels at the sizes where their pipelines can go wrong: odd numbers of 32-k groups, fewer stages than the ring
+holds, ragged rows and columns; the launches that must not depend on timing. Tolerance: assert_gemm_close (one fp16 ulp plus
+the fp32 accumulation-order error, tests/_helpers.py)."""
+import numpy as np
+import pytest
+
+from oracle import hxo
+from tests._helpers import assert_gemm_close, f16
+from tests.test_gpu_kernels import _hip, _q4a_weights, _run_gemm, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(rng, fmt, asym, N, K):
+    wf = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    if fmt == 0:
+        return f16(wf), None, None, f16(wf).view(np.uint16)
+    if asym:
+        q, s, z = _q4a_weights(rng, N, K)
+        return q, s, z, hxo.q4_dequant(q, s, z)
+    q, s = hxo.q8_quantize(wf) if fmt == 1 else hxo.q4_quantize(wf)
+    return q, s, None, hxo.q8_dequant(q, s) if fmt == 1 else hxo.q4_dequant(q, s)
+
+
+FORMATS = [(0, False), (1, False), (2, False), (2, True)]
+
+
+@pytest.mark.parametrize("fmt,asym", FORMATS)
+@pytest.mark.parametrize("K", [32, 64, 96, 160, 288, 352])
+def test_every_tile_at_odd_and_short_k(K, fmt, asym):
+    """One and few 32-k groups, odd and even (stage 0 of an odd count pairs its group with zeros), ragged in M and N: the
+    128x128 tile against the oracle, every other tile equal to it bit for bit (one k order)."""
+    hip = _hip()
+    say(f"tiles fmt={fmt} asym={asym} K={K}")
+    rng = np.random.default_rng(500 + K + 7 * fmt + asym)
+    M, N = 272, 392
+    A = f16(rng.standard_normal((M, K)))
+    q, s, z, wdq = _weights(rng, fmt, asym, N, K)
+    tiles = [(128, 128, 4), (256, 256, 9), (192, 256, 9), (256, 192, 9), (192, 192, 4), (128, 256, 9), (256, 128, 4),
+             (192, 128, 8), (64, 128, 4), (64, 64, 4)] + ([(128, 64, 4)] if fmt != 2 else [])
+    base = _run_gemm(hip, A, fmt, q, s, N, K, tile=tiles[0], z=z)
+    assert_gemm_close(base, hxo.gemm(A, wdq), A, np.asarray(wdq).view(np.float16))
+    for t in tiles[1:]:
+        got = _run_gemm(hip, A, fmt, q, s, N, K, tile=t, z=z)
+        assert np.array_equal(got.view(np.uint16), base.view(np.uint16)), t
+
+
+@pytest.mark.parametrize("fmt,asym", FORMATS)
+@pytest.mark.parametrize("tile", [(256, 192, 9), (192, 192, 4), (64, 128, 4), (64, 64, 4)])
+def test_split_k_of_odd_slices(tile, fmt, asym):
+    """Split-K partials whose slices hold 3 groups each (odd) and 2 (even): each against the oracle over its own slice."""
+    hip = _hip()
+    rng = np.random.default_rng(600 + fmt + asym)
+    M, N = 200, 264
+    for K, S in ((192, 2), (384, 4), (256, 4)):
+        say(f"split-K fmt={fmt} asym={asym} tile={tile} K={K} S={S}")
+        A = f16(rng.standard_normal((M, K)))
+        q, s, z, wdq = _weights(rng, fmt, asym, N, K)
+        w16 = np.asarray(wdq).view(np.float16)
+        got = _run_gemm(hip, A, fmt, q, s, N, K, epi=hip.EPI_PARTIAL, ksplit=S, tile=tile, z=z)
+        for k in range(S):
+            sl = slice(k * K // S, (k + 1) * K // S)
+            Az, Wz = np.ascontiguousarray(A[:, sl]), np.ascontiguousarray(w16[:, sl])
+            assert_gemm_close(got[k], hxo.gemm(Az, Wz.view(np.uint16)), Az, Wz)
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [(1, 1536, 2560, 2560), (0, 512, 2048, 2048), (2, 300, 2048, 2048), (1, 64, 512, 8192)])
+def test_launches_repeat_bit_for_bit(fmt, M, N, K):
+    """40 launches on the same operands give the same bits, whatever runs beside them: a fragment read that the next stage's
+    loads could overtake shows as a difference."""
+    hip = _hip()
+    say(f"repeat fmt={fmt} {M}x{N}x{K}")
+    L = hip.lib()
+    rng = np.random.default_rng(700 + fmt)
+    A = f16(rng.standard_normal((M, K)))
+    q, s, _, _ = _weights(rng, fmt, False, N, K)
+    dA, dW = hip.DeviceArray.from_numpy(A), hip.DeviceArray.from_numpy(q)
+    dS = hip.DeviceArray.from_numpy(s) if s is not None else None
+    for ks in (1, 4):
+        outs = [hip.DeviceArray((ks, M, N), np.float16) for _ in range(8)]
+        first = None
+        for rep in range(5):
+            for o in outs:
+                hip.check(L.hxa_gemm(dA.ptr, K, M, fmt, dW.ptr, dS.ptr if dS else None, None, N, K, ks,
+                                     hip.EPI_PARTIAL if ks > 1 else hip.EPI_STORE, o.ptr, N, M * N, None, 0, None, None, 0, 0,
+                                     None), "gemm")
+            hip.sync()
+            for o in outs:
+                b = o.numpy().view(np.uint16)
+                first = b if first is None else first
+                assert np.array_equal(b, first), (ks, rep)
