@@ -19,7 +19,7 @@ LIB = os.path.join(HERE, "libhexanima_hip.so")
 MOSS_LIB = os.path.join(HERE, "libhexanima_moss.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 PROGRAMS = ["hxa_run", "hxa_blk"]
-SOURCES = ["gemm.hip", "gemm_f16.hip", "gemm_q8.hip", "gemm_q4.hip",
+SOURCES = ["gemm.hip", "gemm_f16.hip", "gemm_q8.hip", "gemm_q4.hip", "gemm_skinny.hip",
            "attention.hip", "elementwise.hip", "runtime.hip", "dit.hip", "noalloc.hip"]
 
 ARCH = os.environ.get("HXA_ARCH", "gfx950")

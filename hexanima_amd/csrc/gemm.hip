@@ -99,6 +99,7 @@ constexpr double kSumLaunchUs = 2.0, kSumBytesPerUs = 12.0e6, kSplitGain = 0.95;
 // tile has one kernel per weight format, whichever of its nw names it
 static bool tile_built(int bm, int bn, int nw, int fmt, bool split2) {
   if (split2) return nw == 4 && bn == 128 && (bm == 128 || bm == 64);
+  if (bn == 32) return nw == 4 && (bm == 64 || bm == 32);  // gemm_skinny.hip: plain stores only (gemm_prepare)
   const bool q4 = fmt == HXA_W_Q4;
   if (nw == 9) return (bn == 256 && (bm == 256 || bm == 192 || bm == 128)) || (bm == 256 && bn == 192) ||
                       ((bm == 128 || bm == 192 || bm == 256) && bn == 128 && !q4);
@@ -215,6 +216,7 @@ static int gemm_prepare(const HxaGemm &g, GemmParams &p, int &bm, int &bn, int &
     nw = g.force_nw ? g.force_nw : 4;
     if (!tile_built(bm, bn, nw, w.fmt, split2)) return HXA_E_ARG;
     if (g.epi == HXA_EPI_SITU && bn % 128 != 0) return HXA_E_ARG;
+    if (bn == 32 && (w.K % 64 != 0 || g.epi != HXA_EPI_STORE || g.ksplit != 1 || p.out_t != nullptr || p.pf_bytes > 0)) return HXA_E_ARG;
     if (headnorm && (bn % 128 != 0 || (p.hn_cols % bn != 0 && p.hn_cols < w.N))) return HXA_E_ARG;
   }
   p.tiles_m = (g.M + bm - 1) / bm;
@@ -261,14 +263,15 @@ int hxa_gemm_launch(const HxaGemm &g, hipStream_t st) {
         ((uintptr_t)sg.x | (uintptr_t)sg.W) % 16)
       return HXA_E_ARG;
     const int ncu = num_cu(), tiles = p.tiles_m * p.tiles_n, idle = (tiles + ncu - 1) / ncu * ncu - tiles;
-    if (tile_nw(bm, bn, w.fmt) == 8 && g.ksplit == 1 && idle >= 16) {
+    if (tile_nw(bm, bn, w.fmt) == 8 && bn > 32 && g.ksplit == 1 && idle >= 16) {
       p.side = sg;
       p.side_wgs = idle;
     } else {
       side_after = true;
     }
   }
-  if (w.fmt == HXA_W_F16) e = launch_fmt<HXA_W_F16, false>(bm, bn, p, g.ksplit, st);
+  if (bn == 32) e = launch_skinny(bm, w.fmt, w.z != nullptr, p, st);
+  else if (w.fmt == HXA_W_F16) e = launch_fmt<HXA_W_F16, false>(bm, bn, p, g.ksplit, st);
   else if (w.fmt == HXA_W_Q8) e = launch_fmt<HXA_W_Q8, false>(bm, bn, p, g.ksplit, st);
   else if (w.z) e = launch_fmt<HXA_W_Q4, true>(bm, bn, p, g.ksplit, st);
   else e = launch_fmt<HXA_W_Q4, false>(bm, bn, p, g.ksplit, st);
@@ -518,9 +521,38 @@ int hxa_sum_partials_launch(const float *p, int S, long zstride, long ldp, int M
   return hipGetLastError() == hipSuccess ? HXA_OK : HXA_E_HIP;
 }
 
-// The K slices hxa_linear runs a linear in: 1 (one launch, fp16 store) or S in {2, 4} (fp32 slices, then their sum)
+// gemm_skinny_kernel's cost model, like kTiles: rounds * (a * K / 1000 + b) + c us, fitted to 16 - 1562 rows x 35 shapes
+// per format (cold weights, row counts up to 3 rounds)
+constexpr struct {
+  int bm;
+  double a[3], b[3], c[3];
+} kSkinny[] = {{64, {2.18, 2.00, 1.96}, {3.19, 3.48, 3.22}, {0.0, 0.0, 0.40}},
+               {32, {1.57, 1.59, 1.62}, {2.52, 2.39, 2.08}, {0.63, 1.05, 1.34}}};
+// the row count (64, 32) of the skinny tile whose modelled time is below t us, else 0
+static int skinny_rows(int M, int N, int K, int fmt, double t) {
+  if (K % 64 != 0) return 0;
+  int bm = 0;
+  for (const auto &c : kSkinny) {
+    const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + 31) / 32), ncu = num_cu();
+    const double ts = (double)((tiles + ncu - 1) / ncu) * (c.a[fmt] * 1e-3 * K + c.b[fmt]) + c.c[fmt];
+    if (ts < t) {
+      t = ts;
+      bm = c.bm;
+    }
+  }
+  return bm;
+}
+int hxa_skinny_rows(int M, int N, int K, int fmt) {
+  fmt &= ~HXA_W_KTILED;
+  if (M <= 0 || N <= 0 || K <= 0 || N % 8 || fmt < 0 || fmt > HXA_W_Q4) return 0;
+  return skinny_rows(M, N, K, fmt, tile_time(M, N, K, 1, fmt));
+}
+// The form hxa_linear runs a linear in. *bm: the rows of gemm_skinny_kernel's tile where its modelled time is within 5% of
+// the other forms' (their model is the more optimistic one: over 105 (M, N, K, format) of 16 - 1562 rows the choice is
+// within 1% of the fastest form, geometric mean; without the skinny kernel 18%), else 0. Result: the K slices, 1 (one launch, fp16 store) or S in {2, 4} (fp32 slices, then their sum)
 // when the tile model's time for S slices plus the slices' round trip through memory is below the one-launch time.
-int hxa_linear_split(int M, int N, int K, int fmt) {
+int hxa_linear_form(int M, int N, int K, int fmt, int *bm) {
+  *bm = 0;
   fmt &= ~HXA_W_KTILED;
   if (M <= 0 || N <= 0 || K <= 0 || N % 8 || fmt < 0 || fmt > HXA_W_Q4) return 1;
   const double t1 = tile_time(M, N, K, 1, fmt);
@@ -536,5 +568,6 @@ int hxa_linear_split(int M, int N, int K, int fmt) {
       best = S;
     }
   }
-  return best;
+  *bm = skinny_rows(M, N, K, fmt, 1.05 * tb);
+  return *bm ? 1 : best;
 }

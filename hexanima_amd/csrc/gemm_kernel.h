@@ -1217,6 +1217,7 @@ hipError_t launch_group_fmt(const GemmParams *ps, int G, int tiles, hipStream_t 
   return hipGetLastError();
 }
 hipError_t launch_xattn(const GemmParams &p, hipStream_t st);  // gemm_f16.hip
+hipError_t launch_skinny(int bm, int fmt, bool asym, const GemmParams &p, hipStream_t st);  // gemm_skinny.hip: bm 32, 64
 
 #define HXG_LAUNCHES(X, FMT, ASYM)                                                                                   \
   X template hipError_t launch_fmt<FMT, ASYM>(int, int, const GemmParams &, int, hipStream_t);                       \

@@ -70,8 +70,11 @@ int hxa_dequant_launch(const HxaWeight &w, hxa_h *out, hipStream_t st);
 // out[m][n] = f16(sum of the S fp32 slices p[z*zstride + m*ldp + n], added in order z = 0 .. S-1)
 int hxa_sum_partials_launch(const float *p, int S, long zstride, long ldp, int M, int N, hxa_h *out, long ldo,
                             hipStream_t st);
-// the K slices hxa_linear runs M x N x K in (1: one launch)
-int hxa_linear_split(int M, int N, int K, int fmt);
+// the K slices hxa_linear runs M x N x K in (1: one launch); *bm: the rows of the one launch's skinny tile (bm x 32,
+// gemm_skinny.hip), 0: the GEMM's own tile choice
+int hxa_linear_form(int M, int N, int K, int fmt, int *bm);
+// the rows of the skinny tile where it is modelled faster than the one-launch GEMM (a plain store), else 0
+int hxa_skinny_rows(int M, int N, int K, int fmt);
 
 struct HxaAttn {
   const hxa_h *q, *k, *vt;  // q [T][ldq], k [NKV][ldk] (head h at column h*128); vt [H*128][ldvt] (keys contiguous)

@@ -230,19 +230,24 @@ extern "C" int hxa_sum_partials(const float *p, int nslice, long zstride, long l
   if (r != HXA_OK) return fail(r, "sum_partials S=%d M=%d N=%d ldp=%ld ldo=%ld rejected", nslice, M, N, ldp, ldo);
   return HXA_OK;
 }
-extern "C" int hxa_linear_split_k(int M, int N, int K, int fmt) { return hxa_linear_split(M, N, K, fmt); }
+extern "C" int hxa_linear_split_k(int M, int N, int K, int fmt) {
+  int bm;
+  return hxa_linear_form(M, N, K, fmt, &bm);
+}
 extern "C" long hxa_linear_ws_bytes(int M, int N, int K, int fmt) {
-  const int ns = hxa_linear_split(M, N, K, fmt);
+  int bm;
+  const int ns = hxa_linear_form(M, N, K, fmt, &bm);
   return ns > 1 ? (long)ns * M * N * 4 : 0;
 }
 extern "C" int hxa_linear(const void *A, long lda, int M, int fmt, const void *w, const void *s, const void *z, int N,
                           int K, void *out, long ldo, void *ws, long ws_bytes, void *stream) {
   if (!out || ldo < N || ldo % 8) return fail(HXA_E_ARG, "linear: output stride %ld for %d columns", ldo, N);
-  const int ns = hxa_linear_split(M, N, K, fmt);
+  int bm;
+  const int ns = hxa_linear_form(M, N, K, fmt, &bm);
   const long need = (long)ns * M * N * 4;
   if (ns == 1 || ws == nullptr || ws_bytes < need)  // one launch, one fp16 rounding of the whole sum
     return gemm_common(A, lda, M, fmt, w, s, z, N, K, 1, HXA_EPI_STORE, out, ldo, 0, nullptr, 0, nullptr, nullptr, 0,
-                       0, 0, 0, 0, stream);
+                       0, bm, bm ? 32 : 0, bm ? 4 : 0, stream);
   TRY(gemm_common(A, lda, M, fmt, w, s, z, N, K, ns, HXA_EPI_PARTIAL_F32, ws, N, (long)M * N, nullptr, 0, nullptr,
                   nullptr, 0, 0, 0, 0, 0, stream));
   return hxa_sum_partials((const float *)ws, ns, (long)M * N, N, M, N, out, ldo, stream);
@@ -887,7 +892,11 @@ int hxa_block_run_chained(const hxa_block_dims *d, const void *pack, float *x, c
   // LoRA-A GEMM (moss blk.c:238, :244, :251, :255): L = f16(a[:, :K] . A^T) into the columns of the same rows right
   // after the K activations (a[:, K:K+N]), where the projection that follows reads it as its last k steps
   auto lora_a = [&](hxa_h *a, long lda, const HxaWeight &A) -> int {
-    return gemm(a, lda, BT, A, HXA_EPI_STORE, a + A.K, lda, nullptr, nullptr, nullptr, 0, 0, 1, 0);
+    HxaGemm g = make(a, lda, BT, A, HXA_EPI_STORE, a + A.K, lda, nullptr, nullptr, nullptr, 0, 0, 1, 0);
+    g.force_bm = hxa_skinny_rows(BT, A.N, A.K, A.fmt);  // 1562 x 8192 -> 128: 49 -> 18 us, x 3072 -> 128: 21 -> 10
+    g.force_bn = g.force_bm ? 32 : 0;
+    const int r = hxa_gemm_launch(g, st);
+    return r == HXA_OK ? r : fail(r, "block LoRA-A gemm N=%d K=%d rejected", A.N, A.K);
   };
   // k groups [g0, g0 + ng) of a k-tiled weight: another k-tiled weight (groups are contiguous slices)
   auto ksub = [](const HxaWeight &w, int g0, int ng) -> HxaWeight {

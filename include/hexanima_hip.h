@@ -152,14 +152,16 @@ int hxa_gemm(const void *A, long lda, int M, int fmt, const void *w, const void 
 /* same, with an explicit tile shape (tests / tuning). Each tile has one kernel per weight format (8 waves above 128x128,
  * 4 or 8 at and below it), under every name that waves gives it: 4 (0 = 4): bm x bn in {192x256, 192x192, 192x128,
  * 256x128, 128x256, 128x128, 64x128, 64x64, 128x64 (not int4)}; 8: {192x256, 192x128, 128x256, 128x128}; 9: {256x256,
- * 192x256, 128x256, 256x192} and, not int4, {256x128, 192x128, 128x128}. SiTU and head norms need bn % 128 == 0. */
+ * 192x256, 128x256, 256x192} and, not int4, {256x128, 192x128, 128x128}. SiTU and head norms need bn % 128 == 0.
+ * 4 also: {64x32, 32x32}, K split over the waves (STORE, ksplit 1, K % 64 == 0). */
 int hxa_gemm_tile(const void *A, long lda, int M, int fmt, const void *w, const void *s, const void *z, int N, int K,
                   int ksplit, int epi, void *out, long ldo, long out_zstride, float *x, long ldx, const float *gate,
                   int bm, int bn, int waves, void *stream);
 /* The plain linear out = f16(A[M][K] . W[N][K]^T) [M][ldo] (gemm_run_ex with STORE, hexagon/mega/gemm2.c:96-141;
  * with int8 / int4 weights the W8A16 / W4A16 linear): one hxa_gemm launch, or, where the tile model favours it (long K,
  * few output tiles: hxa_linear_split_k > 1), that many K slices as fp32 partials in ws (PARTIAL_F32) followed by
- * hxa_sum_partials. The output is rounded to fp16 once either way; only the fp32 summation order differs. ws:
+ * hxa_sum_partials; where 64x32 output tiles leave CUs idle, one launch that splits K over the waves of a workgroup (no
+ * workspace). The output is rounded to fp16 once either way; only the fp32 summation order differs. ws:
  * hxa_linear_ws_bytes(M, N, K, fmt) bytes, 16-byte aligned (NULL or fewer bytes: the one-launch form). Calls that
  * share ws must not overlap. */
 int hxa_linear(const void *A, long lda, int M, int fmt, const void *w, const void *s, const void *z, int N, int K,

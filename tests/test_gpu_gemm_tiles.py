@@ -89,3 +89,63 @@ def test_launches_repeat_bit_for_bit(fmt, M, N, K):
                 b = o.numpy().view(np.uint16)
                 first = b if first is None else first
                 assert np.array_equal(b, first), (ks, rep)
+
+
+@pytest.mark.parametrize("fmt,asym", FORMATS)
+@pytest.mark.parametrize("M,N,K", [(1, 136, 64), (31, 40, 192), (33, 200, 256), (65, 32, 832), (130, 72, 1280), (200, 520, 2048)])
+def test_skinny_tiles(M, N, K, fmt, asym):
+    """The 64x32 and 32x32 tiles with K split over the waves: fewer stages than waves (K = 64, 192), rings that do not fill,
+    ragged rows and columns, a padded output whose padding stays, row-major and k-tiled weights: against the oracle, and the
+    two tiles and layouts bit for bit alike (one wave split, one k order)."""
+    hip = _hip()
+    say(f"skinny fmt={fmt} asym={asym} {M}x{N}x{K}")
+    L = hip.lib()
+    rng = np.random.default_rng(800 + M + K + 7 * fmt + asym)
+    A = f16(rng.standard_normal((M, K)))
+    q, s, z, wdq = _weights(rng, fmt, asym, N, K)
+    kt = hip.ktile(np.ascontiguousarray(q).view(np.uint8).reshape(-1), N, K)
+    dA = hip.DeviceArray.from_numpy(A)
+    dS = hip.DeviceArray.from_numpy(s) if s is not None else None
+    dZ = hip.DeviceArray.from_numpy(z) if z is not None else None
+    ldo, base = N + 8, None
+    for fl, w in ((fmt, q), (fmt | hip.W_KTILED, kt)):
+        dW = hip.DeviceArray.from_numpy(w)
+        for bm in (64, 32):
+            out = hip.DeviceArray.from_numpy(np.full((M, ldo), np.float16(3.0)))
+            hip.check(L.hxa_gemm_tile(dA.ptr, K, M, fl, dW.ptr, dS.ptr if dS else None, dZ.ptr if dZ else None, N, K, 1, 0,
+                                      out.ptr, ldo, 0, None, 0, None, bm, 32, 4, None), "gemm_tile")
+            hip.sync()
+            got = out.numpy()
+            assert np.all(got[:, N:] == np.float16(3.0))
+            got = np.ascontiguousarray(got[:, :N])
+            if base is None:
+                base = got
+                assert_gemm_close(got, hxo.gemm(A, wdq), A, np.asarray(wdq).view(np.float16))
+            assert np.array_equal(got.view(np.uint16), base.view(np.uint16)), (fl, bm)
+    for bad in (dict(K=K - 32), dict(epi=hip.EPI_GELU_TANH), dict(ks=2)):  # whole stages, plain stores, one slice
+        assert L.hxa_gemm_tile(dA.ptr, K, M, fmt, dW.ptr, dS.ptr if dS else None, dZ.ptr if dZ else None, N, bad.get("K", K),
+                               bad.get("ks", 1), bad.get("epi", 0), out.ptr, ldo, 0, None, 0, None, 64, 32, 4, None) != 0
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+def test_linear_takes_the_skinny_tile_for_few_output_tiles(fmt):
+    """hxa_linear at 256 x 2048 x 2048 needs no workspace and gives the 64x32 tile's bits; with K % 64 = 32 it gives the
+    one-launch GEMM's."""
+    hip = _hip()
+    L = hip.lib()
+    rng = np.random.default_rng(900 + fmt)
+    for M, N, K in ((256, 2048, 2048), (64, 256, 544)):
+        say(f"linear fmt={fmt} {M}x{N}x{K}")
+        A = f16(rng.standard_normal((M, K)))
+        q, s, _, _ = _weights(rng, fmt, False, N, K)
+        dA, dW = hip.DeviceArray.from_numpy(A), hip.DeviceArray.from_numpy(q)
+        dS = hip.DeviceArray.from_numpy(s) if s is not None else None
+        sp = dS.ptr if dS else None
+        assert L.hxa_linear_split_k(M, N, K, fmt) == 1 and L.hxa_linear_ws_bytes(M, N, K, fmt) == 0
+        o, t = hip.DeviceArray((M, N), np.float16), hip.DeviceArray((M, N), np.float16)
+        hip.check(L.hxa_linear(dA.ptr, K, M, fmt, dW.ptr, sp, None, N, K, o.ptr, N, None, 0, None), "linear")
+        tile = (64, 32, 4) if K % 64 == 0 else (128, 128, 4)
+        hip.check(L.hxa_gemm_tile(dA.ptr, K, M, fmt, dW.ptr, sp, None, N, K, 1, 0, t.ptr, N, 0, None, 0, None, *tile, None),
+                  "gemm_tile")
+        hip.sync()
+        assert np.array_equal(o.numpy().view(np.uint16), t.numpy().view(np.uint16))
