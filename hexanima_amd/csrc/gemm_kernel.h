@@ -55,7 +55,7 @@ struct GemmParams {
   long pf_bytes;
   HxaClk clk;  // shader-clock record (hxa_clock_record), indexed by the launch's flat workgroup id
   const hxa_h *erf_t2;  // GELU-erf: T2 of every non-negative fp16 bit pattern (null: evaluated in the epilogue)
-  int erf_lds;          // > 0: byte offset in LDS where the epilogue copies the table's first ERF_T2_LDS_N values
+  int erf_lds;          // > 0: byte offset in LDS where the epilogue copies the table from ERF_T2_LDS_LO on
   // fused cross attention (gemm_xattn_kernel): the tile's queries attend to image (m0 / xa_T)'s keys
   // xa_k [NKV][xa_ldk] (+ image * xa_kb), V^T xa_vt [D][xa_ldvt] (+ image * xa_vb); O to xa_o [M][xa_ldo]
   const hxa_h *xa_k, *xa_vt;
@@ -175,9 +175,11 @@ HXA_DEV float gelu_erf_f(float t) {
 // inf patterns included): the GELU-erf epilogue looks its values up instead of evaluating erfcf per output. Filled
 // once per device by erf_t2_kernel with gelu_erf_f's own expression, so a lookup returns the same bits.
 constexpr int ERF_T2_N = 0x8000;
-// the part of the table a GELU-erf epilogue copies into LDS where its tile leaves room: |t| < 6 (bit patterns below
-// 0x4600), 35840 bytes = 35 wave-wide 16-byte copies; larger |t| (rare) is looked up in the global table
-constexpr int ERF_T2_LDS_N = 0x4600, ERF_T2_LDS_BYTES = ERF_T2_LDS_N * 2;
+// the part of the table a GELU-erf epilogue copies into LDS past its tile: 2^-11 <= |t| < 6 (bit patterns 0x1000 to
+// 0x4600), 27648 bytes = 27 wave-wide 16-byte copies, what 256x256 leaves of 160 KB; other |t| (rare) are looked up in the
+// global table. (With the 35 KB of all |t| < 6 the 256x256 tiles had no room and made every lookup from memory: int8 1536 x
+// 2560 x 10240 took 15.2 us longer than with a plain store, now 5.5.)
+constexpr int ERF_T2_LDS_LO = 0x1000, ERF_T2_LDS_N = 0x4600 - ERF_T2_LDS_LO, ERF_T2_LDS_BYTES = ERF_T2_LDS_N * 2;
 HXA_DEV float gelu_erf_tab(float t, const hxa_h *__restrict__ t2tab) {
   const uint32_t b = __builtin_bit_cast(uint16_t, (hxa_h)t) & 0x7fffu;
   return fmaxf(t, 0.0f) - (float)t2tab[b];
@@ -214,7 +216,6 @@ struct GemmGeo {
   static constexpr int lds(int ns) { return ns * STAGE > C_BYTES + PF_LDS ? ns * STAGE : C_BYTES + PF_LDS; }
   // past the staged tile (the ring is dead by then): the touch's sink, then a GELU-erf launch's copy of the T2 table
   static constexpr int PF_OFF = C_BYTES, ERF_OFF = C_BYTES + PF_LDS;
-  static constexpr bool ERF_FITS = ERF_OFF + ERF_T2_LDS_BYTES <= 160 * 1024;
   static constexpr int lds_erf(int ns) {
     return lds(ns) > ERF_OFF + ERF_T2_LDS_BYTES ? lds(ns) : ERF_OFF + ERF_T2_LDS_BYTES;
   }
@@ -368,21 +369,21 @@ HXA_DEV void gemm_epilogue(const GemmParams &p, const hxa_h *Cs, int m0, int n0,
     return;
   }
   }
-  if (p.epi == HXA_EPI_GELU_ERF && p.erf_t2 != nullptr && nsplit == BN) {
+  if (p.epi == HXA_EPI_GELU_ERF && p.erf_lds > 0 && nsplit == BN) {
     // GELU-erf through the T2 table: the LDS reads and table lookups of RB chunks are issued together before any
-    // of them is used, so a thread waits one lookup latency per batch instead of one per chunk. With erf_lds the
-    // table's |t| < 6 part is first copied into LDS past the staged tile (LDS gathers, where global ones issue at
+    // of them is used, so a thread waits one lookup latency per batch instead of one per chunk. The
+    // table's frequent part is first copied into LDS past the staged tile (LDS gathers, where global ones issue at
     // a few lanes per clock)
     constexpr int ITERS = BM * C8 / NT, RB = ITERS % 4 == 0 ? 4 : ITERS % 3 == 0 ? 3 : ITERS % 2 == 0 ? 2 : 1;
     static_assert(BM * C8 % NT == 0 && ITERS % RB == 0, "whole chunk passes");
     static_assert(ERF_T2_LDS_BYTES % 1024 == 0, "whole wave-wide copies");
-    const hxa_h *tl = nullptr;
-    if (p.erf_lds > 0) {
+    const hxa_h *tl;
+    {
       uint8_t *dst = (uint8_t *)Cs + p.erf_lds;
       const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
       for (int c0 = wave * 64; c0 < ERF_T2_LDS_BYTES / 16; c0 += NT) {
         const uint32_t la = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void_t *)(dst + c0 * 16));
-        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p.erf_t2 + (c0 + lane) * 8), "s"(la)
+        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p.erf_t2 + ERF_T2_LDS_LO + (c0 + lane) * 8), "s"(la)
                      : "memory", "m0");
       }
       wait_vm<0>();
@@ -403,7 +404,7 @@ HXA_DEV void gemm_epilogue(const GemmParams &p, const hxa_h *Cs, int m0, int n0,
         for (int e = 0; e < 8; e++) {
           const hxa_h x = v[u][e];  // (a scalar copy: bit_cast of a vector element itself read element 0 only)
           const uint32_t b = __builtin_bit_cast(uint16_t, x) & 0x7fffu;
-          t2[u][e] = tl != nullptr && b < (uint32_t)ERF_T2_LDS_N ? tl[b] : p.erf_t2[b];
+          t2[u][e] = b - ERF_T2_LDS_LO < (uint32_t)ERF_T2_LDS_N ? tl[b - ERF_T2_LDS_LO] : p.erf_t2[b];
         }
       }
 #pragma unroll
@@ -1126,8 +1127,7 @@ hipError_t launch_t(const GemmParams &p, int ksplit, hipStream_t st) {
   auto kern = gemm_kernel<BM, BN, FMT, ASYM, SPLIT2, NW>;
   using G = GemmGeo<BM, BN, FMT>;
   constexpr int base = G::lds(G::NS), lds = SPLIT2 && 2 * G::C_BYTES > base ? 2 * G::C_BYTES : base;
-  constexpr bool erf_ok = !SPLIT2 && G::ERF_FITS;
-  constexpr int most = erf_ok && G::lds_erf(G::NS) > lds ? G::lds_erf(G::NS) : lds;
+  constexpr int most = !SPLIT2 && G::lds_erf(G::NS) > lds ? G::lds_erf(G::NS) : lds;
   static_assert(most <= 160 * 1024, "LDS");
   static bool attr = false;
   if (!attr) {
@@ -1136,7 +1136,7 @@ hipError_t launch_t(const GemmParams &p, int ksplit, hipStream_t st) {
     attr = true;
   }
   const dim3 grid(p.tiles_m * p.tiles_n + (NW == 8 && !SPLIT2 && ksplit == 1 ? p.side_wgs : 0), 1, ksplit);
-  if (erf_ok && p.epi == HXA_EPI_GELU_ERF && p.erf_t2 != nullptr) {  // the T2 table past the staged tile
+  if (!SPLIT2 && p.epi == HXA_EPI_GELU_ERF && p.erf_t2 != nullptr) {  // the T2 table past the staged tile
     GemmParams pe = p;
     pe.erf_lds = G::ERF_OFF;
     hxa_launch(kern, grid, dim3(64 * NW), most, st, pe);

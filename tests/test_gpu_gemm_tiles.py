@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import hxo
-from tests._helpers import assert_gemm_close, f16
+from tests._helpers import assert_gemm_close, f16, ulp_diff
 from tests.test_gpu_kernels import _hip, _q4a_weights, _run_gemm, say
 
 pytestmark = pytest.mark.gpu
@@ -149,3 +149,23 @@ def test_linear_takes_the_skinny_tile_for_few_output_tiles(fmt):
                   "gemm_tile")
         hip.sync()
         assert np.array_equal(o.numpy().view(np.uint16), t.numpy().view(np.uint16))
+
+
+@pytest.mark.parametrize("tile", [(256, 256, 9), (192, 256, 9), (128, 128, 4), (64, 64, 4)])
+def test_gelu_erf_over_every_fp16_value(tile):
+    """GELU-erf of every finite fp16 value and of infinities and NaN, which the LDS part of the lookup table (2^-11 <= |t| < 6)
+    and the global one share: within 2 ulps of the oracle (the fp16 rounding of T2 and of the result), the oracle's NaNs."""
+    hip = _hip()
+    say(f"gelu erf tile={tile}")
+    M, N, K = 256, 256, 32
+    vals = np.arange(65536, dtype=np.uint16).view(np.float16).reshape(M, N)
+    # one launch per 32 columns: A[m][k] = vals[m][32 j + k], W[n] = e_(n % 32)
+    W = f16(np.tile(np.eye(32), (N // 32, 1)))
+    for j in range(0, N // 32):
+        A = vals[:, 32 * j:32 * j + 32].copy()
+        bad = ~np.isfinite(A).all(axis=1)  # inf * 0: the whole row is NaN
+        got = _run_gemm(hip, A, 0, W, None, N, K, epi=hip.EPI_GELU_ERF, tile=tile)[:, :32]
+        t = np.where(np.isfinite(A), A, np.float16(0))
+        ref = hxo.gelu(t, 0).view(np.float16)
+        assert ulp_diff(np.ascontiguousarray(got[~bad]), np.ascontiguousarray(ref[~bad])).max() <= 2
+        assert np.isnan(got[bad]).all()
