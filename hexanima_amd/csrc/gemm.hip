@@ -89,6 +89,9 @@ static double tile_time(int M, int N, int K, int ksplit, int fmt) {
   }
   return 1e30;
 }
+double hxa_gemm_model_us(int M, int N, int K, int fmt, int ksplit) {
+  return tile_time(M, N, K, ksplit, fmt & ~HXA_W_KTILED);
+}
 // split-K linear cost terms: the sum kernel's launch (us) and the bytes per us of the slices' round trip through L2 /
 // MALL, fitted with the gain below to one launch, two and four slices timed on 258 (M, N, K, format) of 16 - 4096 rows
 // (geometric mean of choice / fastest form 1.008; the worst 1.42, fp16 544 x 12288 -> 3072); kSplitGain: the

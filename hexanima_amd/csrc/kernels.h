@@ -55,6 +55,8 @@ int hxa_gemm_xattn_launch(const HxaGemm &g, const HxaXAttn &a, hipStream_t st);
 // whether the fused kernel's 128 x 128 tiles of an M x N projection fit in one round over the CUs (beyond one round
 // the projection's own tile pick plus the attention kernel is faster)
 bool hxa_gemm_xattn_fits(int M, int N);
+// the modelled time (us) of a plain-store GEMM M x N x K in ksplit slices (a slice's partial as a store)
+double hxa_gemm_model_us(int M, int N, int K, int fmt, int ksplit);
 // whether hxa_gemm_pair_launch(g0, g1) would be one launch that takes no more rounds of workgroups over the CUs than
 // g0 alone (g1 only fills CUs g0 leaves idle)
 bool hxa_gemm_pair_fits(const HxaGemm &g0, const HxaGemm &g1);

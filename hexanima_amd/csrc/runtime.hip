@@ -498,24 +498,28 @@ struct WsLayout {
   long dq_bytes;            // size of WS_DQ's first slot (0: no quantised projection is dequantised first)
   long dq2_off, dq2_bytes;  // its second slot (text k / v weight)
 };
-// Quantised cross-q projections (and, from DQ_WIDE_ROWS rows, every quantised projection) at this many rows or more
-// run as one dequantisation pass into fp16 (WS_DQ) and the fp16 kernels; below DQ_WIDE_ROWS the attention-output and
-// MLP-down projections run fused split-K 4 (q_split4), the wider ones (qkv, MLP up) fused on their own tiles.
-constexpr long DQ_MIN_ROWS = 1024;
-// from this many rows on the pass also pays for the wide projections (qkv, MLP up / up-gate)
-constexpr long DQ_WIDE_ROWS = 4096;
-// int8 / int4 attention-output and MLP-down projections at DQ_MIN_ROWS .. DQ_WIDE_ROWS rows (no LoRA) run fused,
-// split-K 4 on the 8-wave tiles, into four fp16 partials that the next norm adds: those tiles hide the
-// dequantisation under their MFMAs, and no fp16 copy of the weight goes through memory (1536 tokens, 2.9B-class
-// MLP-down 10240 -> 2560: 80 us fused against 15.5 us of dequantisation + 84.5 us of fp16 GEMM in the step).
-// Not with the reference's rounding points (round_ref: mega_block), which round o once and the MLP-down in two halves.
-static bool q_split4(const hxa_block_dims *d, int fmt, int K) {
+// From this many rows on every int8 / int4 projection runs as one dequantisation pass into fp16 (WS_DQ) and the fp16
+// kernels; below, the GEMM dequantises under its MFMAs. Measured, int8, pass + fp16 against direct (us): 1024 x 2048 -> 2048
+// 20.4 / 18.5, 1568 x 3200 -> 3072 46.6 / 42.3, 4096 x 2048 -> 8192 128.6 / 125.7, 6656 x 3072 -> 3072 128.0 / 133.7, 6656 x
+// 12288 -> 3072 512 / 520; int4 at 6656 rows 1 - 9% in favour of the pass.
+constexpr long DQ_ROWS = 4096;
+// The fused cross attention takes fp16 weights only: from this many rows on its cross-q projection goes through the pass.
+constexpr long XDQ_ROWS = 1024;
+// int8 / int4 attention-output and MLP-down projections (K -> D) at 1024 .. DQ_ROWS - 1 rows run in 2 or 4 K slices, fp16
+// partials that the next norm adds; 0: not this form. Four slices where the tile model saves more on the GEMM than two more
+// partials cost to write and read back (1536 rows: 10240 -> 2560 83.5 us in two slices, 78.0 in four; 2560 -> 2560 26.2 and
+// 27.5, and the norm that adds them 10 and 13).
+// Not with the reference's rounding points (round_ref: mega_block), which round o once and the MLP-down in two halves; not
+// with the LoRA's o, whose one pass is as fast.
+static int q_parts(const hxa_block_dims *d, int fmt, int K) {
   const long BT = (long)d->batch * d->T;
-  return d->kind != 2 && !d->round_ref && (fmt & ~HXA_W_KTILED) != HXA_W_F16 && BT >= DQ_MIN_ROWS && BT < DQ_WIDE_ROWS &&
-         K % 128 == 0;
+  if (d->kind == 2 || d->round_ref || (fmt & ~HXA_W_KTILED) == HXA_W_F16 || BT < 1024 || BT >= DQ_ROWS || K % 128 != 0)
+    return 0;
+  const double extra = 8.0 * BT * d->D / 8.0e6;  // us: two more partials out and in at 8 TB/s (L2 / MALL)
+  return hxa_gemm_model_us((int)BT, d->D, K, fmt, 4) + extra < hxa_gemm_model_us((int)BT, d->D, K, fmt, 2) ? 4 : 2;
 }
-// fp16 partials the MLP-down leaves (pending across a chain of blocks): 4 in the fused split-K 4 form, else 2
-int hxa_block_down_parts(const hxa_block_dims *d) { return q_split4(d, d->fmt_mlp, d->F) ? 4 : 2; }
+// fp16 partials the MLP-down leaves (pending across a chain of blocks): 2 or 4
+int hxa_block_down_parts(const hxa_block_dims *d) { return q_parts(d, d->fmt_mlp, d->F) == 4 ? 4 : 2; }
 static WsLayout ws_layout(const hxa_block_dims *d) {
   const long BT = (long)d->batch * d->T, BC = (long)d->batch * d->C, D = d->D;
   // with the LoRA (kind 2) the rows of h, o and mid carry the L columns of the projection that reads them:
@@ -534,7 +538,7 @@ static WsLayout ws_layout(const hxa_block_dims *d) {
   L.ld[WS_K] = 2 * D;
   put(WS_VT, 2 * D * BT, BT);
   put(WS_O, 2 * BT * LDO, LDO);
-  const long nparts = q_split4(d, d->fmt_attn, d->D) || hxa_block_down_parts(d) == 4 ? 4 : 2;
+  const long nparts = q_parts(d, d->fmt_attn, d->D) == 4 || hxa_block_down_parts(d) == 4 ? 4 : 2;
   put(WS_T1, 2 * nparts * BT * D, D);  // split-K partials, BT x D apart
   L.off[WS_T2] = L.off[WS_T1] + 2 * BT * D;
   L.ld[WS_T2] = D;
@@ -546,20 +550,18 @@ static WsLayout ws_layout(const hxa_block_dims *d) {
     L.off[WS_CK] = L.off[WS_CVT] = 0;
     L.ld[WS_CK] = L.ld[WS_CVT] = 0;
   }
-  // fp16 copy of the largest int8 / int4 projection weight that runs through the dequantisation pass: from
-  // DQ_MIN_ROWS rows those with N <= K (attention output, cross q, MLP down), from DQ_WIDE_ROWS rows all of them
+  // fp16 copy of the largest int8 / int4 projection weight that runs through the dequantisation pass: from DQ_ROWS rows
+  // all of them, from XDQ_ROWS rows the cross q
   const MatList mats = pack_mats(d->kind, d->D, d->F, d->DC, d->fmt_attn, d->fmt_mlp);
   const int nproj = d->kind == 0 ? 7 : 4;  // the LoRA-A matrices run fused
   long dq = 0;
-  for (int i = 0; i < nproj && BT >= DQ_MIN_ROWS; i++) {
+  for (int i = 0; i < nproj; i++) {
     const MatSpec &m = mats.m[i];
     if (m.fmt == HXA_W_F16 || (d->kind == 0 && i == 3)) continue;  // the text k / v weight has its own slot
-    const bool o_like = i == 1 || (d->kind == 0 && i == 4), down = i == (d->kind == 0 ? 6 : 3);
-    if ((o_like && q_split4(d, m.fmt, m.K)) || (down && q_split4(d, m.fmt, m.K))) continue;  // fused split-K 4
-    if (BT >= DQ_WIDE_ROWS || m.N <= m.K) dq = std::max(dq, 2L * m.N * m.K);
+    if (BT >= DQ_ROWS || (d->kind == 0 && i == 2 && BT >= XDQ_ROWS)) dq = std::max(dq, 2L * m.N * m.K);
   }
   // a second slot for the text k / v weight (2D x DC), so that it and the cross q run as one paired fp16 launch
-  const long dq2 = d->kind == 0 && d->fmt_attn != HXA_W_F16 && BT >= DQ_MIN_ROWS ? al256(2 * 2 * D * (long)d->DC) : 0;
+  const long dq2 = d->kind == 0 && d->fmt_attn != HXA_W_F16 && BT >= DQ_ROWS ? al256(2 * 2 * D * (long)d->DC) : 0;
   put(WS_DQ, al256(dq) + dq2, d->F);
   L.dq_bytes = dq;
   L.dq2_off = al256(dq);
@@ -705,7 +707,7 @@ int hxa_block_textkv_plan(const hxa_block_dims *d, const void *pack, const void 
                           HxaGemm *g, HxaWeight *w) {
   if (d->kind != 0 || check_dims(d) != HXA_OK || !pack || !ctx || !ck || !cvt || !g || !w) return 0;
   const long BT = (long)d->batch * d->T, BC = (long)d->batch * d->C, D = d->D;
-  if (BT >= DQ_WIDE_ROWS || d->T % 128 || d->C % 8) return 0;
+  if (BT >= DQ_ROWS || d->T % 128 || d->C % 8) return 0;
   const PackView pv = pack_view(d, pack);
   const HxaWeight &Wqkv = pv.w[0], &Wcq = pv.w[2], &Wckv = pv.w[3];
   const float *gain = pv.vec;
@@ -727,7 +729,7 @@ int hxa_block_textkv_plan(const hxa_block_dims *d, const void *pack, const void 
   kv.hn_g0 = kv.hn_g1 = gain + 384;
   kv.hn_gsplit = (int)D;
   kv.hn_ttab = d->T;
-  // the qkv projection as the runner launches it below DQ_WIDE_ROWS rows (its own weights, head norm + RoPE, V^T);
+  // the qkv projection as the runner launches it below DQ_ROWS rows (its own weights, head norm + RoPE, V^T);
   // only its shape and tile matter here
   HxaGemm qkv = kv;
   qkv.A = ck;
@@ -843,16 +845,14 @@ int hxa_block_run_chained(const hxa_block_dims *d, const void *pack, float *x, c
     g.split_col = split;
     return g;
   };
-  // the weight a projection runs on: w itself, or (int8 / int4, N <= K, WS_DQ sized) its fp16 k-tiled copy made
+  // the weight a projection runs on: w itself, or (int8 / int4 from min_rows rows, WS_DQ sized) its fp16 k-tiled copy made
   // now in WS_DQ. One copy at a time: each is consumed by the launch that follows it on this stream.
   HxaWeight wdq{};
   HxaWeight wdq2{};
-  auto prep = [&](const HxaWeight &w, const HxaWeight *&wp, int slot = 0) -> int {
+  auto prep = [&](const HxaWeight &w, const HxaWeight *&wp, int slot = 0, long min_rows = DQ_ROWS) -> int {
     wp = &w;
     const int f = w.fmt & ~HXA_W_KTILED;
-    if (f == HXA_W_F16 || BT < DQ_MIN_ROWS) return HXA_OK;
-    if (slot == 0 && ((w.N > w.K && BT < DQ_WIDE_ROWS) || 2L * w.N * w.K > L.dq_bytes)) return HXA_OK;
-    if (slot == 1 && 2L * w.N * w.K > L.dq2_bytes) return HXA_OK;
+    if (f == HXA_W_F16 || BT < min_rows || 2L * w.N * w.K > (slot ? L.dq2_bytes : L.dq_bytes)) return HXA_OK;
     hxa_h *buf = (hxa_h *)(w8 + L.off[WS_DQ] + (slot ? L.dq2_off : 0));
     const int r = hxa_dequant_launch(w, buf, st);
     if (r != HXA_OK) return fail(r, "block dequant N=%d K=%d rejected", w.N, w.K);
@@ -909,19 +909,18 @@ int hxa_block_run_chained(const hxa_block_dims *d, const void *pack, float *x, c
   // split-K down projection + gated residual (blk.c:172-174): two fp16 partial GEMMs over 2x the workgroups (fills
   // the GPU at N = D) then the residual; measured faster than the single-launch HXA_EPI_RESADD_SPLIT2 form, whose
   // 128-wide tiles leave a quarter of the CUs idle at 1536 x 2048. With the LoRA the halves are [0, F/2) and
-  // [F/2, F) + the LoRA columns (moss blk.c:256-259): two launches.
+  // [F/2, F) + the LoRA columns (moss blk.c:256-259): two launches where the rounding points are the reference's or a stage
+  // is dumped, else two equal slices of F + the LoRA columns in one (1562 x 8320 -> 3072 int8: 110 us with its
+  // dequantisation pass -> 92).
   // with a stage stop the MLP-down runs in the reference's two K halves (the dumped t holds the first half's partial,
   // blk.c:172-173) whatever the workspace layout allows
   const int down_np = stop ? 2 : hxa_block_down_parts(d);
   auto down_resadd = [&](const hxa_h *a, const HxaWeight &w, const float *gate) -> int {
     const HxaWeight *wp = &w;
-    if (down_np == 4) {
-      TRY(gemm(a, ldmid, BT, w, HXA_EPI_PARTIAL, t1, D, nullptr, nullptr, nullptr, 0, 0, 4, (long)BT * D));
-    } else if (!lora) {
-      TRY(prep(w, wp));
-      TRY(gemm(a, ldmid, BT, *wp, HXA_EPI_PARTIAL, t1, D, nullptr, nullptr, nullptr, 0, 0, 2, (long)BT * D));
+    TRY(prep(w, wp));
+    if (!lora || (!stop && !d->round_ref && w.K % 64 == 0)) {
+      TRY(gemm(a, ldmid, BT, *wp, HXA_EPI_PARTIAL, t1, D, nullptr, nullptr, nullptr, 0, 0, down_np, (long)BT * D));
     } else {
-      TRY(prep(w, wp));
       const int G = F / 64;  // k groups of one half
       const HxaWeight w0 = ksub(*wp, 0, G), w1 = ksub(*wp, G, G + LORA_R / 32);
       TRY(gemm(a, ldmid, BT, w0, HXA_EPI_STORE, t1, D, nullptr, nullptr, nullptr, 0, 0, 1, 0));
@@ -934,14 +933,13 @@ int hxa_block_run_chained(const hxa_block_dims *d, const void *pack, float *x, c
   // prologue and epilogue a large share -- two fp16 K-half partials into t1 and t2 on twice the workgroups, which
   // the norm adds (1536 tokens: 4% faster for fp16, 9-21% for int8 / int4 weights; slower on a grid of 192x256 or
   // 256x256 tiles or of several rounds). split_o says which.
-  // int8 / int4 weights at 1024 .. 4095 rows: the fused split-K 4 form (q_split4), four partials. o_np: the partials
-  // the next norm adds.
+  // int8 / int4 weights at 1024 .. DQ_ROWS - 1 rows: q_parts partials. o_np: the partials the next norm adds.
   bool split_o = false;
   int o_np = 1;
   auto deferred_proj = [&](const HxaWeight &w) -> int {
-    if (q_split4(d, w.fmt, w.K) && !stop) {
-      o_np = 4;
-      return gemm(o, ldo, BT, w, HXA_EPI_PARTIAL, t1, D, nullptr, nullptr, nullptr, 0, 0, 4, (long)BT * D);
+    if (const int qp = stop ? 0 : q_parts(d, w.fmt, w.K)) {
+      o_np = qp;
+      return gemm(o, ldo, BT, w, HXA_EPI_PARTIAL, t1, D, nullptr, nullptr, nullptr, 0, 0, qp, (long)BT * D);
     }
     const HxaWeight *wp;
     TRY(prep(w, wp));
@@ -1043,7 +1041,7 @@ int hxa_block_run_chained(const hxa_block_dims *d, const void *pack, float *x, c
       // projection is one head's 128 queries, which attend to their image's text keys from LDS
       hn = HeadNorm{D, gain + 256, gain + 256, D, nullptr, nullptr};
       const HxaWeight *wcq;
-      TRY(prep(Wcq, wcq));
+      TRY(prep(Wcq, wcq, 0, XDQ_ROWS));
       const HxaGemm gq = make(h, ldh, BT, *wcq, HXA_EPI_STORE, qk, ldqk, nullptr, nullptr, nullptr, 0, 0, 1, 0);
       const HxaXAttn xa{ck, cvT, o, D, BC, ldo, (long)d->C * D, d->C, d->C, d->C, T};
       int r = hxa_gemm_xattn_launch(gq, xa, st);
