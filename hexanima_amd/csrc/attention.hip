@@ -10,10 +10,13 @@
 // halves are merged through LDS at the end. (96 queries on 6 waves would fill 256 CUs at 1536 queries x 16 heads,
 // but waves are dealt to the SIMDs round-robin, two SIMDs then run two waves, and the workgroup takes as long as
 // the 128-query one: 29.5 against 29.0 us on MI355X.) Each wave owns 32
-// queries and keeps Q in registers. Two schedules of the key loop: lock-step (one barrier per tile for both halves)
-// and, for whole tiles in a multiple of 4, ping-pong (each tile split into a VALU phase, the softmax, and an MFMA
+// queries and keeps Q in registers. Schedules of the key loop: lock-step (one barrier per tile for both halves); for whole
+// tiles in an even number ping-pong (each tile split into a VALU phase, the softmax, and an MFMA
 // phase, PV with the next QK; the halves one phase apart, so the two waves of a SIMD alternate between the two
-// kinds of work: 5-6% faster at 1536 and 6656 keys on MI355X).
+// kinds of work: 5-6% faster at 1536 and 6656 keys on MI355X); and with 2 x 6 waves, 192 queries, three-phase (softmax, PV
+// and the next QK as phases of the three waves of a SIMD). What bounds them all is the softmax's VALU phase (about 1000
+// issue cycles per 32 x 64 scores, half of them v_exp_f32) and, beside it, LDS reads near 128 B / clk; queries_per_wg
+// chooses the workgroup that wastes least of the last round.
 //
 // Per 64-key tile a wave computes S^T = K . Q^T (v_mfma_f32_32x32x16_f16), so a lane holds 16 scores of ONE query
 // and the row max needs a single exchange between the wave's two halves (v_permlane32_swap). K rows are stored in LDS with rows 4-7 and 8-11 of every 16 swapped,
@@ -47,9 +50,12 @@ HXA_DEV float16_t mfma(half8_t a, half8_t b, float16_t c) { return __builtin_amd
 // masking and no clamped per-lane tile addresses. PF: the launch touches weights for the next kernel (p.pf_bytes > 0). Both are compile-time so that the
 // main loop holds only the code it runs: the general form kept 44 - 62 scalar registers spilled to VGPR lanes and
 // their v_readlane / v_writelane in the loop.
-template <int NWH, bool FULL, bool PF, bool PP = false>
-__global__ __launch_bounds__(2 * NWH * 64) void attn_kernel(HxaAttn p, int nqb) {
+// SCHED: the schedule of the key loop, 0 lock-step, 1 ping-pong, 2 three-phase (NWH = 6).
+template <int NWH, bool FULL, bool PF, int SCHED = 0>
+__global__ __launch_bounds__(2 * NWH * 64, 2) void attn_kernel(HxaAttn p, int nqb) {
+  constexpr bool PP = SCHED == 1;
   static_assert(!PP || FULL, "the ping-pong form runs whole tiles only");
+  static_assert((SCHED == 2) == (NWH == 6), "three waves a SIMD: three phases");
   constexpr int QB = NWH * 32;  // queries per workgroup
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -88,11 +94,12 @@ __global__ __launch_bounds__(2 * NWH * 64) void attn_kernel(HxaAttn p, int nqb) 
   // waves of the half. Keys past NKV read a valid row (their probability is 0).
   // A tile that lies wholly below NKV moves only a wave-uniform base: each lane's byte offsets within the tile are
   // fixed (koff / voff, computed once), so those loads take the scalar-base form with no per-lane address math.
-  constexpr int NLD = (16 + NWH - 1) / NWH;
-  uint32_t koff[NLD], voff[NLD];
+  // (of 6 waves the first 4 load: blocks 4 apart differ by a uniform 16 keys or 32 rows of V^T, so one offset serves all)
+  constexpr int NWL = NWH == 6 ? 4 : NWH, NLD = (16 + NWL - 1) / NWL, NOFF = NWH == 6 ? 1 : NLD;
+  uint32_t koff[NOFF], voff[NOFF];
 #pragma unroll
-  for (int j = 0; j < NLD; j++) {
-    const int blk = min(j * NWH + wq, 15);
+  for (int j = 0; j < NOFF; j++) {
+    const int blk = min(j * NWL + wq, 15);
     const int row = 4 * blk + (lane >> 4), c = (lane & 15) ^ (row & 15);
     koff[j] = ((uint32_t)krow_key(row) * (uint32_t)p.ldk + c * 8) * 2u;
     const int d = 8 * blk + (lane >> 3), cv = (lane & 7) ^ ((d >> 1) & 7);
@@ -102,48 +109,49 @@ __global__ __launch_bounds__(2 * NWH * 64) void attn_kernel(HxaAttn p, int nqb) 
   // form's loads past the last tile, into a buffer that is never read again)
   auto load_kv = [&](int i, bool with_k, bool with_v, int src = -1) {
     const int key0 = (t0 + (src >= 0 ? src : i)) * KT;
+    if (NWL < NWH && wq >= NWL) return;
     if (FULL || key0 + KT <= p.NKV) {
       if (with_k) {
         const hxa_h *kt = k + (long)key0 * p.ldk;
 #pragma unroll
         for (int j = 0; j < NLD; j++) {
-          const int blk = j * NWH + wq;
-          if (16 % NWH == 0 || blk < 16) g2l16_sbase(kt, koff[j], kbuf(i) + blk * 1024);
+          const int blk = j * NWL + wq;
+          if (16 % NWL == 0 || blk < 16) g2l16_sbase(NOFF == 1 ? kt + (long)j * 16 * p.ldk : kt, koff[NOFF == 1 ? 0 : j], kbuf(i) + blk * 1024);
         }
       }
       if (with_v) {
         const hxa_h *vtt = vt + key0;
 #pragma unroll
         for (int j = 0; j < NLD; j++) {
-          const int blk = j * NWH + wq;
-          if (16 % NWH == 0 || blk < 16) g2l16_sbase(vtt, voff[j], vbuf(i) + blk * 1024);
+          const int blk = j * NWL + wq;
+          if (16 % NWL == 0 || blk < 16) g2l16_sbase(NOFF == 1 ? vtt + (long)j * 32 * p.ldvt : vtt, voff[NOFF == 1 ? 0 : j], vbuf(i) + blk * 1024);
         }
       }
       return;
     }
     if constexpr (FULL) return;
+    // the tile that ends past NKV; the lane is opaque here so that the loop keeps none of its addresses in registers
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
     if (with_k) {
-      uint8_t *dst = kbuf(i);
 #pragma unroll
-      for (int j = 0; j < (16 + NWH - 1) / NWH; j++) {
-        const int blk = j * NWH + wq;
-        if (16 % NWH == 0 || blk < 16) {
-          const int row = 4 * blk + (lane >> 4), c = (lane & 15) ^ (row & 15);
-          const int key = min(key0 + krow_key(row), p.NKV - 1);
-          g2l16_opaque(k + (long)key * p.ldk + c * 8, dst + blk * 1024);
+      for (int j = 0; j < NLD; j++) {
+        const int blk = j * NWL + wq;
+        if (16 % NWL == 0 || blk < 16) {
+          const int row = 4 * blk + (ln >> 4), c = (ln & 15) ^ (row & 15);
+          const int key = min(krow_key(row), p.NKV - 1 - key0);
+          g2l16_sbase(k + (long)key0 * p.ldk, ((uint32_t)key * (uint32_t)p.ldk + c * 8) * 2u, kbuf(i) + blk * 1024);
         }
       }
     }
     if (with_v) {
-      uint8_t *dst = vbuf(i);
 #pragma unroll
-      for (int j = 0; j < (16 + NWH - 1) / NWH; j++) {
-        const int blk = j * NWH + wq;
-        if (16 % NWH == 0 || blk < 16) {
-          const int d = 8 * blk + (lane >> 3), c = (lane & 7) ^ ((d >> 1) & 7);
-          int key = key0 + c * 8;
-          if (key >= p.NKV) key = 0;
-          g2l16_opaque(vt + (long)d * p.ldvt + key, dst + blk * 1024);
+      for (int j = 0; j < NLD; j++) {
+        const int blk = j * NWL + wq;
+        if (16 % NWL == 0 || blk < 16) {
+          const int d = 8 * blk + (ln >> 3), c = (ln & 7) ^ ((d >> 1) & 7);
+          const int key = key0 + c * 8 < p.NKV ? c * 8 : 0;
+          g2l16_sbase(vt + key0, ((uint32_t)d * (uint32_t)p.ldvt + key) * 2u, vbuf(i) + blk * 1024);
         }
       }
     }
@@ -412,6 +420,147 @@ __global__ __launch_bounds__(2 * NWH * 64) void attn_kernel(HxaAttn p, int nqb) 
     mphase(nh - 1, std::false_type{});  // the last tile: no next QK
     bar();
     if (half == 0) bar();  // the last phase: half 1's M(nh - 1)
+  } else if constexpr (SCHED == 2) {
+    // Three-phase form: each tile is three phases, V(i) = its softmax (VALU), P(i) = its PV, Q(i) = the QK of tile i+1
+    // (MFMA, half the work of a tile each), and the three waves of a SIMD (w, w + 4, w + 8) run one phase apart, so in
+    // every phase one of them computes exponentials while the other two fill the matrix core. Wave group ph = wave / 4
+    // runs V(i), P(i), Q(i) in the phases 3 i + ph, 3 i + 1 + ph, 3 i + 2 + ph; one workgroup barrier per phase.
+    //  V^T(i) is read in the phases 3 i + 1 .. 3 i + 3, K(i + 1) in 3 i + 2 .. 3 i + 4, so phase g = 3 j + 1 issues
+    //  V^T(j + 1) and g = 3 j + 2 issues K(j + 2), each into the buffer whose last reader finished a phase earlier. At the
+    //  end of phase 3 j (3 j + 1) a wave waits for its V^T(j) (K(j + 1)) loads: all but the youngest 4, which are
+    //  those of the K (V^T) tile after them (waves that load nothing have nothing to wait for).
+    const int ph = wave >> 2, nph = 3 * nh + 2;
+    half8_t pf[2][2];
+    auto begin = [&](int g) {  // the loads of phase g
+      const int j = g / 3, r = g - 3 * j;
+      if (r == 1) {
+        if (j + 1 < nmine) load_kv(j + 1, false, true);
+        if (PF && j < pf_steps) touch(j);
+      } else if (r == 2 && j + 2 < nmine) {
+        load_kv(j + 2, true, false);
+      }
+    };
+    // LDS byte offsets of this lane's fragments within a tile: V^T (dblk, kk) at (vrow ^ (kk << 5)) + dblk * 4096, K (ds,
+    // kb2) at (krow ^ (ds << 5)) + kb2 * 8192; opaque per phase, or the twelve XORed values would be kept in registers
+    uint32_t vrow = ql * 128 + ((g ^ ((ql >> 1) & 7)) << 4), krow = ql * 256 + ((g ^ (ql & 15)) << 4);
+    auto end = [&](int g) {
+      const int r = g % 3;
+      if (r != 2) {
+        // past the half's last loads nothing younger is in flight: wait for all
+        if (g / 3 + 2 < nmine) wait_vm<4>();
+        else wait_vm<0>();
+      }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr int AH = 2;  // fragment reads in flight ahead of the MFMAs (6 in P and 4 in Q: no faster)
+    auto pphase = [&](int i) {
+      const uint8_t *vb = vbuf(i);
+      asm volatile("" : "+v"(vrow));
+      auto frag = [&](int j) {  // j = kk * 4 + dblk, kk = kb2 * 2 + ks
+        return *(const half8_t *)(vb + (vrow ^ ((j >> 2) << 5)) + (j & 3) * 4096);
+      };
+      half8_t fr[AH + 1];
+#pragma unroll
+      for (int j = 0; j < AH; j++) fr[j] = frag(j);
+#pragma unroll
+      for (int j = 0; j < 16; j++) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (j + AH < 16) fr[(j + AH) % (AH + 1)] = frag(j + AH);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[j & 3] = mfma(fr[j % (AH + 1)], pf[j >> 3][(j >> 2) & 1], acc[j & 3]);
+      }
+    };
+    auto qphase = [&](int i) {  // S = K Q^T of tile i
+      const uint8_t *kb = kbuf(i);
+      asm volatile("" : "+v"(krow));
+      auto frag = [&](int j) {  // j = ds * 2 + kb2
+        return *(const half8_t *)(kb + (krow ^ ((j >> 1) << 5)) + (j & 1) * 8192);
+      };
+      Sa[0] = (float16_t){};
+      Sa[1] = (float16_t){};
+      half8_t fr[AH + 1];
+#pragma unroll
+      for (int j = 0; j < AH; j++) fr[j] = frag(j);
+#pragma unroll
+      for (int j = 0; j < 16; j++) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (j + AH < 16) fr[(j + AH) % (AH + 1)] = frag(j + AH);
+        __builtin_amdgcn_sched_barrier(0);
+        Sa[j & 1] = mfma(fr[j % (AH + 1)], qf[j >> 1], Sa[j & 1]);
+      }
+    };
+    auto vphase = [&](int i) {
+      const int key0 = (t0 + i) * KT;
+      if (!FULL && key0 + KT > p.nvalid) {
+        const int lim = p.nvalid - key0 - 8 * g;
+#pragma unroll
+        for (int kb2 = 0; kb2 < 2; kb2++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            Sa[kb2][r] = kb2 * 32 + 16 * (r >> 3) + (r & 7) < lim ? Sa[kb2][r] : -INFINITY;
+            if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+          }
+      }
+      float m4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+      for (int kb2 = 0; kb2 < 2; kb2++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) m4[r & 3] = fmaxf(m4[r & 3], Sa[kb2][r]);
+      float mt = fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3]));
+      {
+        float lo, hi;
+        halves(mt, lo, hi);
+        mt = fmaxf(lo, hi);
+      }
+      const bool need = mt > mrun + RESCALE_TH;  // also when mrun is still -inf
+      if (__any(need)) {
+        const float alpha = need ? __builtin_amdgcn_exp2f((mrun - mt) * L2E) : 1.0f;
+        if (need) mrun = mt;
+        lsum *= alpha;
+#pragma unroll
+        for (int d = 0; d < 4; d++) acc[d] *= alpha;
+      }
+      const float mb = (mrun == -INFINITY ? 0.0f : mrun) * L2E;
+      float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int idx = 0; idx < 32; idx += 2) {
+        const int kb2 = idx >> 4, r = idx & 15;
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(Sa[kb2][r], L2E, -mb));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(Sa[kb2][r + 1], L2E, -mb));
+        const half2_t h2 = {(hxa_h)p0, (hxa_h)p1};
+        pf[kb2][r >> 3][r & 7] = h2[0];
+        pf[kb2][r >> 3][(r & 7) + 1] = h2[1];
+        ls[(idx >> 1) & 3] = __builtin_amdgcn_fdot2(h2, (half2_t){(hxa_h)1.0f, (hxa_h)1.0f}, ls[(idx >> 1) & 3], false);
+      }
+      lsum += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+    };
+    // (every wave's QK of tile 0 has to be done before phase 2 loads K(2) over it: the barriers of phases 0 and 1)
+    int g3 = 0;
+    for (; g3 < ph; g3++) {
+      begin(g3);
+      end(g3);
+    }
+    for (int i = 0; i < nh; i++) {
+      // (the else branches end the lives of P and S: 48 registers that the compiler would carry through the phases)
+      begin(g3);
+      if (i < nmine) vphase(i);
+      else pf[0][0] = pf[0][1] = pf[1][0] = pf[1][1] = (half8_t){};
+      end(g3++);
+      begin(g3);
+      if (i < nmine) pphase(i);
+      end(g3++);
+      begin(g3);
+      if (i + 1 < nmine) qphase(i + 1);
+      else Sa[0] = Sa[1] = (float16_t){};
+      end(g3++);
+    }
+    for (; g3 < nph; g3++) {
+      begin(g3);
+      end(g3);
+    }
   } else {
     for (int i = 0; i < nh; i += 2) {
       step(i, Sa, Sb);
@@ -531,6 +680,35 @@ __global__ __launch_bounds__(256) void attn_short_kernel(HxaAttn p, int nqb) {
   store_rows32(lds + 8 * TILE_BYTES + wave * 8192, v, lane, o + (long)row0 * p.ldo, p.ldo, p.T - row0);
 }
 
+// CUs of the device current at the first call (0: unknown)
+int attn_ncu() {
+  static const int ncu = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return 0;
+    return n > 0 ? n : 0;
+  }();
+  return ncu;
+}
+// The ping-pong form takes whole tiles, as many in either half.
+bool ping_pong(int nvalid) { return nvalid % (2 * KT) == 0; }
+// Queries per workgroup of a launch past 256 keys.
+// 64 (4 waves, ping-pong) where their grid fits in one round: half the queries per SIMD, and twice the CUs (512 queries x 16
+// heads, 128 workgroups instead of 64: 12.8 -> 11.0 us; 1024 x 16 18.7 -> 16.5; as the second round begins it loses, 1536 x
+// 16 26.0 -> 38.6).
+// 192 (12 waves, three-phase): a round takes about 1.45 times as long as one of 128 (12 key tiles a half: 39.4 us, 30.1),
+// so where they save more than a third of the rounds (1568 x 24: 216 workgroups in one round instead of 312 in two, 58.2 ->
+// 43.5 us; 3072 x 16: 256 instead of 384, 89.4 -> 81.6). With as many rounds, or 4 instead of 5, they are slower (6656 x 24:
+// 511 -> 618).
+// 128 otherwise.
+int queries_per_wg(int T, int H, int batch, int nvalid) {
+  const long ncu = attn_ncu(), hb = (long)H * batch;
+  if (ncu == 0) return 128;
+  if (ping_pong(nvalid) && (T + 63) / 64 * hb <= ncu) return 64;
+  const long r4 = ((T + 127) / 128 * hb + ncu - 1) / ncu, r6 = ((T + 191) / 192 * hb + ncu - 1) / ncu;
+  return 3 * r6 < 2 * r4 ? 192 : 128;
+}
+
 }  // namespace
 
 int hxa_attn_launch(const HxaAttn &p, hipStream_t st) {
@@ -557,17 +735,22 @@ int hxa_attn_launch(const HxaAttn &p, hipStream_t st) {
     const HxaSideGemv &g = p.side;
     return hxa_modgemv_launch(g.x, g.K, g.W, g.N, g.y, g.per, g.ostride, g.split, g.gap, g.act, st);
   };
+  constexpr int LDS = LDS_BYTES + SINK_BYTES;
+  constexpr int LDS6 = 6 * (66 * 64 * 4 + 8192);  // the merge and the output staging of 12 waves: more than the tiles
+  static_assert(LDS6 >= LDS && LDS6 <= 160 * 1024, "LDS");
   static bool attr = false;
   if (!attr) {
-    const void *kerns[] = {(const void *)attn_kernel<4, false, false>,      (const void *)attn_kernel<4, false, true>,
-                           (const void *)attn_kernel<4, true, false>,       (const void *)attn_kernel<4, true, true>,
-                           (const void *)attn_kernel<4, true, false, true>, (const void *)attn_kernel<4, true, true, true>};
-    for (const void *kf : kerns)
-      if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES + SINK_BYTES) != hipSuccess)
-        return HXA_E_HIP;
-    if (hipFuncSetAttribute((const void *)attn_short_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SK_LDS) !=
-        hipSuccess)
-      return HXA_E_HIP;
+    const struct {
+      const void *f;
+      int lds;
+    } kerns[] = {{(const void *)attn_kernel<4, false, false>, LDS},    {(const void *)attn_kernel<4, false, true>, LDS},
+                 {(const void *)attn_kernel<4, true, false>, LDS},     {(const void *)attn_kernel<4, true, true>, LDS},
+                 {(const void *)attn_kernel<4, true, false, 1>, LDS},  {(const void *)attn_kernel<4, true, true, 1>, LDS},
+                 {(const void *)attn_kernel<2, true, false, 1>, LDS},  {(const void *)attn_kernel<2, true, true, 1>, LDS},
+                 {(const void *)attn_kernel<6, false, false, 2>, LDS6}, {(const void *)attn_kernel<6, false, true, 2>, LDS6},
+                 {(const void *)attn_short_kernel, SK_LDS}};
+    for (const auto &k : kerns)
+      if (hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, k.lds) != hipSuccess) return HXA_E_HIP;
     attr = true;
   }
   HxaAttn pk = p;
@@ -581,36 +764,39 @@ int hxa_attn_launch(const HxaAttn &p, hipStream_t st) {
     if (hipGetLastError() != hipSuccess) return HXA_E_HIP;
     return side_alone();
   }
-  const int nqb = (p.T + 127) / 128;
-  const bool full = p.nvalid % KT == 0, pf = p.pf_bytes > 0;
-  dim3 grid(nqb * p.H + p.side_wgs, p.batch);
-  const int lds = LDS_BYTES + SINK_BYTES;
-  // the ping-pong form: whole tiles, the same even number of tiles in both halves (HXA_ATTN_PP=0: lock-step form)
+  // (HXA_ATTN_PP=0: the lock-step form in the place of the ping-pong one)
   static const int pp_env = [] {
     const char *e = getenv("HXA_ATTN_PP");
     return e ? atoi(e) : 1;
   }();
-  if (pp_env && full && (p.nvalid / KT) % 4 == 0) {
-    pf ? hxa_launch(attn_kernel<4, true, true, true>, grid, dim3(512), lds, st, pk, nqb)
-       : hxa_launch(attn_kernel<4, true, false, true>, grid, dim3(512), lds, st, pk, nqb);
-    return hipGetLastError() == hipSuccess ? HXA_OK : HXA_E_HIP;
-  }
-  if (full) pf ? hxa_launch(attn_kernel<4, true, true>, grid, dim3(512), lds, st, pk, nqb)
-            : hxa_launch(attn_kernel<4, true, false>, grid, dim3(512), lds, st, pk, nqb);
-  else pf ? hxa_launch(attn_kernel<4, false, true>, grid, dim3(512), lds, st, pk, nqb)
-          : hxa_launch(attn_kernel<4, false, false>, grid, dim3(512), lds, st, pk, nqb);
+  const bool full = p.nvalid % KT == 0, pf = p.pf_bytes > 0, pp = pp_env && ping_pong(p.nvalid);
+  int qb = queries_per_wg(p.T, p.H, p.batch, p.nvalid);
+  if (qb == 64 && !pp) qb = 128;
+  const int nqb = (p.T + qb - 1) / qb;
+  const dim3 grid(nqb * p.H + p.side_wgs, p.batch);
+  if (qb == 192)
+    pf ? hxa_launch(attn_kernel<6, false, true, 2>, grid, dim3(768), LDS6, st, pk, nqb)
+       : hxa_launch(attn_kernel<6, false, false, 2>, grid, dim3(768), LDS6, st, pk, nqb);
+  else if (qb == 64)
+    pf ? hxa_launch(attn_kernel<2, true, true, 1>, grid, dim3(256), LDS, st, pk, nqb)
+       : hxa_launch(attn_kernel<2, true, false, 1>, grid, dim3(256), LDS, st, pk, nqb);
+  else if (pp)
+    pf ? hxa_launch(attn_kernel<4, true, true, 1>, grid, dim3(512), LDS, st, pk, nqb)
+       : hxa_launch(attn_kernel<4, true, false, 1>, grid, dim3(512), LDS, st, pk, nqb);
+  else if (full)
+    pf ? hxa_launch(attn_kernel<4, true, true>, grid, dim3(512), LDS, st, pk, nqb)
+       : hxa_launch(attn_kernel<4, true, false>, grid, dim3(512), LDS, st, pk, nqb);
+  else
+    pf ? hxa_launch(attn_kernel<4, false, true>, grid, dim3(512), LDS, st, pk, nqb)
+       : hxa_launch(attn_kernel<4, false, false>, grid, dim3(512), LDS, st, pk, nqb);
   return hipGetLastError() == hipSuccess ? HXA_OK : HXA_E_HIP;
 }
 
 int hxa_attn_idle_wgs(int T, int H, int batch) {
   if (batch != 1 || T <= 0 || H <= 0) return 0;
-  static const int ncu = [] {  // CUs of the device current at the first call (0: unknown, no side GEMV)
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      return 0;
-    return n > 0 ? n : 0;
-  }();
+  const int ncu = attn_ncu();
   if (ncu == 0) return 0;
-  const int ntot = (T + 127) / 128 * H, rem = ntot % ncu, idle = rem == 0 ? 0 : ncu - rem;
+  const int qb = queries_per_wg(T, H, batch, T);
+  const int ntot = (T + qb - 1) / qb * H, rem = ntot % ncu, idle = rem == 0 ? 0 : ncu - rem;
   return idle >= ncu / 4 ? idle : 0;
 }
