@@ -153,8 +153,8 @@ def test_anima_block_stages_and_batch():
                                                       (6656, 6656, 64, 96, 12288, 512, 1e-2)])
 def test_moss_block_joint_attention_q8_q4(T, nv, gh, gw, F, ntxt, maxabs):
     """MOSS-class block (joint attention with a key mask, RMS-mod, SiTU, int8 attention / int4 MLP weights). At
-    1088 rows the int8 o projection and the int4 MLP-down run through the fp16 dequantisation pass, at 4128 rows
-    every projection does. The last case is config 4's own block: 6144 image tokens (64 x 96) + 512 text tokens,
+    1088 rows the GEMMs dequantise as they run, at 4128 rows every projection goes through the fp16 dequantisation
+    pass. The last case is config 4's own block: 6144 image tokens (64 x 96) + 512 text tokens,
     D 3072, 24 heads, SiTU FFN 12288 (up-gate N = 24576)."""
     hip = _hip()
     say(f"moss block T={T} nvalid={nv} D=3072 F={F} q8/q4")
@@ -209,8 +209,8 @@ def lora_pack_mats(rng, D, F, fmt_attn, fmt_mlp):
 def test_moss_lora_block_q8_q4(T, nv, gh, gw):
     """MOSS-class block with the rapid-moss LoRA (kind-2 pack: moss/hexagon/mega/blk.c:238-259): four LoRA-A GEMMs
     write L next to the activations they read, and every projection runs on [x | L] . [W ; s B] with the B rows as 4
-    extra k groups; the down projection's second K half carries them. int8 attention / int4 MLP weights; at 1088
-    rows the o and down projections, at 4128 rows all of them, run through the dequantisation pass."""
+    extra k groups; the down projection's second K half carries them. int8 attention / int4 MLP weights; at 4128
+    rows every projection but the LoRA-A runs through the dequantisation pass."""
     hip = _hip()
     say(f"moss LoRA block T={T} nvalid={nv} D=3072 F=4096 q8/q4")
     rng = np.random.default_rng(13)
@@ -744,7 +744,7 @@ def test_dit_side_gemv_matches_separate_modulation(D, H, F, fmt, lat_hw, monkeyp
     kernels: the latents after four steps equal, bit for bit, those with every modulation in its own launches
     (HXA_DIT_SIDE=0). 2B at 1536 tokens: 192 attention workgroups host the GEMV in appended workgroups; at 192
     tokens the attention runs the short-key kernel and the GEMV its own launch after it; 2.9B-class int8 at 1536
-    tokens: the qkv and MLP-up ping-pong grids (240 workgroups each) host half of the rows each; 2B at 2048 tokens:
+    tokens: the qkv and MLP-up grids (240 workgroups each) host half of the rows each; 2B at 2048 tokens:
     the attention fills the CUs (256 workgroups), the qkv launch is paired with the text k / v (its half of the rows
     then runs as its own launch) and the MLP-up grid hosts its half in a second, partly filled round."""
     hip = _hip()

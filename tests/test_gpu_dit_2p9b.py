@@ -4,7 +4,7 @@ caller-side glue of phone/animad.cpp:424-492 around them.
 
 At this shape the qkv grid leaves no room for the text k / v tiles in its own launch, so the runner computes every
 block's text k / v up front in one grouped launch and each block fuses its cross q with the attention; the
-attention-output and MLP-down projections run fused split-K 4 into four fp16 partials. The oracle dequantises the
+attention-output and MLP-down projections run in two and four K slices, fp16 partials that the next norm adds. The oracle dequantises the
 same int8 weights (f16(q s), gemm2.c:19-35) and computes in double with the reference block's rounding points.
 Tolerance about 3x the error measured on MI355X, as the other DiT tests."""
 import ctypes as C_
@@ -22,7 +22,7 @@ LAT = (16, 96, 64)
 
 
 # weight format (0 fp16, 1 int8, 2 int4) and bounds: the fp16 and int4 forms take the same grouped text k / v launch
-# (the qkv grid is the same 240 tiles); int4 runs its attention-output and MLP-down projections fused split-K 4 too
+# (the qkv grid is the same 240 tiles); int4 runs its attention-output and MLP-down projections in K slices too
 @pytest.mark.parametrize("fmt,tol", [(1, (2e-3, 9e-3)), (0, (2e-3, 9e-3)), (2, (2e-3, 9e-3))])
 def test_dit_2p9b_two_blocks_velocity_vs_oracle(fmt, tol):
     from hexanima_amd import hip

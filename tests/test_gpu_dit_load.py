@@ -60,7 +60,7 @@ def mgl1_bin(tensors):
     return np.frombuffer(bytes(buf), np.uint8).copy()
 
 
-# 256 image tokens, and the benchmark's 1536 (a 96 x 64 latent; int8 blocks then take the fused split-K 4 form)
+# 256 image tokens, and the benchmark's 1536 (a 96 x 64 latent; int8 blocks then run their outputs in K slices)
 @pytest.mark.parametrize("q8,LAT", [(False, (16, 32, 32)), (True, (16, 32, 32)), (False, (16, 96, 64)),
                                     (True, (16, 96, 64))])
 def test_dit_anima_from_blk_files_and_small_bin(q8, LAT):

@@ -56,7 +56,7 @@ def _run_gemm(hip, A, fmt, w, s, N, K, epi=0, ksplit=1, tile=None, x=None, gate=
     return dx.numpy() if resadd else out.numpy()
 
 
-# waves 9: the ping-pong 8-wave kernel
+# (a tile has one kernel per weight format, whichever wave count names it)
 @pytest.mark.parametrize("tile", [None, (192, 256), (192, 256, 8), (192, 192), (192, 128), (256, 128), (128, 256), (128, 128),
                                   (64, 128), (128, 64), (192, 256, 9), (256, 256, 9), (128, 256, 9), (128, 128, 9)])
 def test_gemm_f16_tiles(tile):
@@ -275,7 +275,7 @@ def test_gelu_epilogues_every_fp16_input():
                                       if not (f == 2 and t == (128, 128, 9))])
 def test_gemm_partial_split_k_tiles(fmt, tile):
     """Split-K into two fp16 partials (the K halves of the MLP-down and of the deferred attention-output projection)
-    on the ping-pong, 8-wave and 4-wave tiles for each weight format: each half is the oracle GEMM of its K half;
+    on 8-wave and 4-wave tiles for each weight format: each half is the oracle GEMM of its K half;
     M and N ragged against the tiles."""
     hip = _hip()
     say(f"gemm partial ksplit=2 fmt={fmt} tile={tile}")
@@ -479,8 +479,8 @@ def _attn(hip, q, k, v, nvalid=None, batch=1):
 # tile short
 # the last case is the MOSS-class joint attention at its own shape (6144 image + 512 text tokens, 24 heads); the
 # oracle (rows are independent) is evaluated on a sample of 416 query rows spread over all key tiles' range.
-# Whole key tiles in a multiple of 4 (1536, 6656, 1024 over 1000 ragged queries, and 512 over 200) take the
-# ping-pong form: the key halves one phase apart; 320 keys on 5 tiles and 384 keys on 6 do not qualify
+# Whole key tiles in an even number (1536, 6656, 1024 over 1000 ragged queries, 512 over 200, 384) take the
+# ping-pong form: the key halves one phase apart; 320 keys on 5 tiles do not qualify
 @pytest.mark.parametrize("T,NKV,nvalid,H", [(1536, 1536, 1536, 16), (1536, 256, 256, 16), (448, 448, 430, 4), (96, 64, 64, 2),
                                             (1024, 1024, 1000, 32), (300, 512, 500, 3), (200, 576, 520, 2),
                                             (200, 512, 512, 3), (96, 320, 320, 2), (6656, 6656, 6656, 24),
@@ -801,7 +801,7 @@ def test_sum_partials_exact():
 @pytest.mark.parametrize("fmt,tile", [(f, t) for f in (0, 1, 2)
                                       for t in (None, (128, 128, 4), (192, 128, 4), (128, 256, 8), (192, 256, 9),
                                                 (128, 128, 9))
-                                      if not (f == 2 and t == (128, 128, 9))])  # (no int4 ping-pong 128x128 kernel)
+                                      if not (f == 2 and t == (128, 128, 9))])  # (no such name with int4)
 def test_gemm_partial_f32_slices(fmt, tile):
     """PARTIAL_F32: each of 4 K slices' fp32 sums (no fp16 rounding) against the oracle's double-accumulated GEMM
     over that slice, within the fp32 accumulation bound 4 sqrt(K/4) 2^-24 sum|a w| + 2^-24 |ref|; ragged M and N."""

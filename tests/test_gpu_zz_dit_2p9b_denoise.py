@@ -5,13 +5,13 @@ reference block's rounding points, blk.c:149-176, with the weights dequantised a
 with the caller-side glue of phone/animad.cpp:424-492), with the same weights (exported from the GPU runner).
 
 At this shape the runner takes its fast forms: every block's text k / v in one grouped launch before the chain, the
-cross q fused with its attention, and the attention-output, cross-output and MLP-down projections fused split-K 4 into
-four fp16 partials (four roundings where the reference rounds o once and the MLP-down in two halves). This test
+cross q fused with its attention, and the attention-output, cross-output and MLP-down projections in two or four K
+slices, fp16 partials (up to four roundings where the reference rounds o once and the MLP-down in two halves). This test
 measures how those extra roundings compound over the 112 block evaluations of the denoise.
 
 Tolerance: the reference's own block metric (cmp_block.py:5-6) on the whole denoise, rel err on the latent change and
 cosine, plus max abs, at about 3x the error measured on MI355X (4.9e-4 and 2.3e-3, the same as the 2B fp16 denoise's
-5.3e-4 and 2.4e-3: the split-K 4 partials' extra roundings do not compound measurably). The oracle needs about two minutes on 16 host
+5.3e-4 and 2.4e-3: the partials' extra roundings do not compound measurably). The oracle needs about two minutes on 16 host
 threads; progress is printed after every step. Collected after the other GPU tests."""
 import ctypes as C_
 import time
