@@ -450,10 +450,7 @@ __global__ __launch_bounds__(2 * NWH * 64, 2) void attn_kernel(HxaAttn p, int nq
         if (g / 3 + 2 < nmine) wait_vm<4>();
         else wait_vm<0>();
       }
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
+      reads_done_barrier();
     };
     constexpr int AH = 2;  // fragment reads in flight ahead of the MFMAs (6 in P and 4 in Q: no faster)
     auto pphase = [&](int i) {

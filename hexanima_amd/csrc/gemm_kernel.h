@@ -598,10 +598,7 @@ HXA_DEV void xattn_tail(const GemmParams &p, const float4_t (&acc)[NI][MI], int 
   for (int i = 0; i < ntiles; i++) {
     if (i + 1 < ntiles) wait_vm<8>();  // tile i landed (tile i + 1 may still fly)
     else wait_vm<0>();
-    // a plain barrier (no fence): tile i + 1's loads stay in flight
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    reads_done_barrier();  // (tile i + 1's loads stay in flight)
     const uint8_t *kb = kbuf(i), *vb = vbuf(i);
     // every K fragment of the tile, then the V^T fragments, read ahead of the MFMAs that use them (the V^T reads
     // land during the QK MFMAs and the softmax)
@@ -670,9 +667,7 @@ HXA_DEV void xattn_tail(const GemmParams &p, const float4_t (&acc)[NI][MI], int 
     for (int j = 0; j < 16; j++)
       o[j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[j], pf[j >> 3][(j >> 2) & 1], o[j & 3], 0, 0, 0);
     if (i + 2 < ntiles) {
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_s_barrier();  // every wave's reads of buffer i & 1 are in registers (the MFMAs used them)
-      asm volatile("" ::: "memory");
+      reads_done_barrier();  // buffer i & 1 has been read by every wave
       xattn_load_kv(p, m0, n0, i + 2, wave, lane, lds8);
     }
   }
@@ -1016,11 +1011,7 @@ HXA_DEV void gemm_body(const GemmParams &p, const int bid, const int z) {
   // stage t + 1 landed for every wave, and this wave's LDS reads are in registers
   auto stage_barrier = [&]() {
     wait_vm<(NS - 2) * LMIN>();
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
+    reads_done_barrier();
   };
   [[maybe_unused]] half4_t first[SPLIT2 ? NI : 1][SPLIT2 ? MI : 1];
   auto half_done = [&](int t) {

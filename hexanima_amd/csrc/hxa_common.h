@@ -121,6 +121,16 @@ HXA_DEV void wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
+// A workgroup barrier behind which LDS that this wave has read may be loaded over: the reads are waited for (they may still be
+// queued when their MFMAs stand behind the barrier, and another wave's load would overtake them), and nothing moves across.
+// Outstanding direct loads are not waited for, as __syncthreads would.
+HXA_DEV void reads_done_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
 // 16 bytes per lane from global memory straight into LDS: lane l writes lds_base + 16 l
 HXA_DEV void g2l16(const void *g, void *lds_base) {
   __builtin_amdgcn_global_load_lds((gmem_void_t *)g, (lds_void_t *)lds_base, 16, 0, 0);
