@@ -697,11 +697,15 @@ bool ping_pong(int nvalid) { return nvalid % (2 * KT) == 0; }
 // so where they save more than a third of the rounds (1568 x 24: 216 workgroups in one round instead of 312 in two, 58.2 ->
 // 43.5 us; 3072 x 16: 256 instead of 384, 89.4 -> 81.6). With as many rounds, or 4 instead of 5, they are slower (6656 x 24:
 // 511 -> 618).
-// 128 otherwise.
-int queries_per_wg(int T, int H, int batch, int nvalid) {
+// 128 otherwise. A launch that hosts a side GEMV (hosts) never takes 64: that form occupies twice the CUs and its appended
+// workgroups have 4 waves, so the GEMV's 50 MB are streamed by half as many waves or fewer (768 x 16: 256 instead of 1280) and
+// outlast the attention (2B step per block, fp16, 64 against 128 queries: 512 tokens 174.4 / 172.7 us, 768 215.6 / 207.9, 1024,
+// where 64 leave no CU to host on, 231.8 / 228.0; 2.9B class, 640 tokens: 289.1 / 267.0). 192 host as well as 128 (2304 x 16:
+// 433.6, with 128 451.1).
+int queries_per_wg(int T, int H, int batch, int nvalid, bool hosts) {
   const long ncu = attn_ncu(), hb = (long)H * batch;
   if (ncu == 0) return 128;
-  if (ping_pong(nvalid) && (T + 63) / 64 * hb <= ncu) return 64;
+  if (!hosts && ping_pong(nvalid) && (T + 63) / 64 * hb <= ncu) return 64;
   const long r4 = ((T + 127) / 128 * hb + ncu - 1) / ncu, r6 = ((T + 191) / 192 * hb + ncu - 1) / ncu;
   return 3 * r6 < 2 * r4 ? 192 : 128;
 }
@@ -767,7 +771,7 @@ int hxa_attn_launch(const HxaAttn &p, hipStream_t st) {
     return e ? atoi(e) : 1;
   }();
   const bool full = p.nvalid % KT == 0, pf = p.pf_bytes > 0, pp = pp_env && ping_pong(p.nvalid);
-  int qb = queries_per_wg(p.T, p.H, p.batch, p.nvalid);
+  int qb = queries_per_wg(p.T, p.H, p.batch, p.nvalid, p.side_wgs > 0);
   if (qb == 64 && !pp) qb = 128;
   const int nqb = (p.T + qb - 1) / qb;
   const dim3 grid(nqb * p.H + p.side_wgs, p.batch);
@@ -793,7 +797,7 @@ int hxa_attn_idle_wgs(int T, int H, int batch) {
   if (batch != 1 || T <= 0 || H <= 0) return 0;
   const int ncu = attn_ncu();
   if (ncu == 0) return 0;
-  const int qb = queries_per_wg(T, H, batch, T);
+  const int qb = queries_per_wg(T, H, batch, T, true);
   const int ntot = (T + qb - 1) / qb * H, rem = ntot % ncu, idle = rem == 0 ? 0 : ncu - rem;
   return idle >= ncu / 4 ? idle : 0;
 }

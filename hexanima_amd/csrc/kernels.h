@@ -97,7 +97,7 @@ struct HxaAttn {
   int side_wgs = 0;
 };
 int hxa_attn_launch(const HxaAttn &p, hipStream_t st);
-// workgroups an attention launch of T queries x H heads (batch 1) leaves idle on this GPU: what side_wgs may use
+// workgroups an attention launch of T queries x H heads (batch 1) that hosts a side GEMV leaves idle: what side_wgs may use
 // (0 when the tiles leave fewer than a quarter of the CUs idle in their last round: too few to stream a GEMV in
 // the attention's time)
 int hxa_attn_idle_wgs(int T, int H, int batch);

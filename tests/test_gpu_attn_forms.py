@@ -1,5 +1,7 @@
 """The attention kernel's workgroup sizes and schedules at the edges of their ranges, against the oracle's exact softmax with
 the bounds of test_gpu_kernels.test_attention_vs_oracle (fp16 P and output rounding, about 3x the measured errors)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -39,3 +41,38 @@ def test_attention_forms(T, NKV, nvalid, H, batch):
         exact = exact.view(np.float16).astype(np.float64)
         assert np.max(np.abs(g - exact)) < 4e-3
         assert rel(g, exact) < 1e-3
+
+
+@pytest.mark.parametrize("lat_hw,wgs,alone", [((64, 32), 64, 128), ((64, 48), 96, 192)])
+def test_attention_that_hosts_the_modulation_keeps_128_queries(lat_hw, wgs, alone, monkeypatch):
+    """2B-class DiT at 512 and 768 tokens, batch 1: the self-attention launch that streams the next block's modulation runs in
+    128-query workgroups (8 waves each, the CUs it leaves idle host the rows); with the modulation in its own launches
+    (HXA_DIT_SIDE=0) in 64-query ones. Counted from the clock record each attention workgroup writes; the latents are the same
+    bits either way."""
+    hip = _hip()
+    L = hip.lib()
+    say(f"hosting attention lat {lat_hw}")
+    rng = np.random.default_rng(12)
+    lat = rng.standard_normal((1, 16) + lat_hw).astype(np.float32)
+    ctx = rng.standard_normal((1, 256, 1024)).astype(np.float32)
+    outs = []
+    for side, want in (("1", wgs), ("0", alone)):
+        monkeypatch.setenv("HXA_DIT_SIDE", side)
+        rec = hip.DeviceArray((1024, 4), np.uint64, zero=True)
+        bd = hip.BlockDims(0, 2048, 16, 8192, 256, 1024, 0, 1, 0, 0, 0, 1)
+        cfg = hip.DitCfg(bd, 2, 16, lat_hw[0], lat_hw[1], 256, 0)
+        p = C.c_void_p()
+        hip.check(L.hxa_dit_create(C.byref(cfg), 77, C.byref(p)), "dit_create")
+        try:
+            hip.check(L.hxa_clock_record(1, rec.ptr, 1024), "clock_record")
+            hip.check(L.hxa_dit_set_inputs(p, lat.ctypes.data, ctx.ctypes.data), "set_inputs")
+            hip.check(L.hxa_dit_step(p, 1.0, 0.5, 1), "step")
+            cur = np.zeros_like(lat)
+            hip.check(L.hxa_dit_get_latent(p, cur.ctypes.data), "get")
+        finally:
+            L.hxa_clock_record(1, None, 0)
+            L.hxa_dit_destroy(p)
+        assert np.count_nonzero(rec.numpy()[:, 0]) == want
+        outs.append(cur)
+    assert np.abs(outs[0] - lat).max() > 0.1
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
