@@ -174,8 +174,12 @@ static int gemm_prepare(const HxaGemm &g, GemmParams &p, int &bm, int &bn, int &
     p.w_rs = wkt ? cb : (long)w.K / 32 * cb;
     p.w_gs = wkt ? cb * w.N : cb;
   }
-  // the loaders' per-lane offsets within a tile (up to 256 rows) are 32-bit: keep them below 2^31
-  if (g.lda >= (1L << 22) || p.w_rs * (w.fmt == HXA_W_F16 ? 2 : 1) >= (1L << 23) || w.N >= (1 << 24)) return HXA_E_ARG;
+  // the loaders' per-lane offsets within a stage (up to 256 rows, two k groups) are unsigned 32-bit
+  {
+    const long es = w.fmt == HXA_W_F16 ? 2 : 1;
+    if (g.lda >= (1L << 22) || p.w_rs * es >= (1L << 23)) return HXA_E_ARG;
+    if ((255 * p.w_rs + p.w_gs + 32) * es >= (1L << 32) || 4L * w.N >= (1L << 32)) return HXA_E_ARG;
+  }
   p.M = g.M;
   p.N = w.N;
   p.Ktot = w.K;

@@ -169,3 +169,43 @@ def test_gelu_erf_over_every_fp16_value(tile):
         ref = hxo.gelu(t, 0).view(np.float16)
         assert ulp_diff(np.ascontiguousarray(got[~bad]), np.ascontiguousarray(ref[~bad])).max() <= 2
         assert np.isnan(got[bad]).all()
+
+
+@pytest.mark.parametrize("fmt,N", [(0, 2**24 + 264), (1, 2**24 + 264), (2, 2**24 + 264), (0, 2**25 + 1032)])
+def test_linear_of_many_columns(fmt, N):
+    """k-tiled weights whose second k group lies 2^28 to 2^31 bytes and more behind the first, where the loaders' 32-bit offsets
+    have to reach it: the first and last 264 columns against the oracle."""
+    hip = _hip()
+    say(f"linear fmt={fmt} N={N}")
+    L = hip.lib()
+    M, K, n = 8, 96, 264
+    rng = np.random.default_rng(1000 + fmt)
+    A = f16(rng.standard_normal((M, K)))
+    dA, out = hip.DeviceArray.from_numpy(A), hip.DeviceArray((M, N), np.float16)
+    unit = (64, 32, 16)[fmt]
+    dW = hip.DeviceArray((K // 32 * N * unit,), np.uint8)
+    cols = []  # the weights of both ends, the rest stays what a fill leaves
+    hip.check(L.hxa_fill_normal(dW.ptr, 1, K // 32 * N * unit // 2, 5, 0.0, 0.05, None), "fill")
+    dS = None
+    if fmt:
+        dS = hip.DeviceArray((K // 32, N), np.float16)
+        hip.check(L.hxa_fill_const(dS.ptr, 1, K // 32 * N, 1e-3, None), "fill")
+    hip.sync()
+    for n0 in (0, N - n):
+        q, s, _, wdq = _weights(rng, fmt, False, n, K)
+        kt = hip.ktile(np.ascontiguousarray(q).view(np.uint8).reshape(-1), n, K).reshape(K // 32, n * unit)
+        for g in range(K // 32):
+            row = np.ascontiguousarray(kt[g])
+            hip.check(L.hxa_h2d(dW.at((g * N + n0) * unit), row.ctypes.data, row.nbytes), "h2d")
+            if fmt:
+                sr = np.ascontiguousarray(np.asarray(s).reshape(K // 32, n)[g])
+                hip.check(L.hxa_h2d(dS.at((g * N + n0) * 2), sr.ctypes.data, sr.nbytes), "h2d")
+        cols.append((n0, np.asarray(wdq).view(np.float16)))
+    hip.check(L.hxa_linear(dA.ptr, K, M, fmt | hip.W_KTILED, dW.ptr, dS.ptr if dS else None, None, N, K, out.ptr, N, None, 0,
+                           None), "linear")
+    hip.sync()
+    for n0, w in cols:
+        got = np.zeros((M, n), np.float16)
+        for m in range(M):
+            hip.check(L.hxa_d2h(got[m:].ctypes.data, out.at((m * N + n0) * 2), 2 * n), "d2h")
+        assert_gemm_close(got, hxo.gemm(A, w.view(np.uint16)), A, w)
