@@ -209,3 +209,26 @@ def test_linear_of_many_columns(fmt, N):
         for m in range(M):
             hip.check(L.hxa_d2h(got[m:].ctypes.data, out.at((m * N + n0) * 2), 2 * n), "d2h")
         assert_gemm_close(got, hxo.gemm(A, w.view(np.uint16)), A, w)
+
+
+@pytest.mark.parametrize("asym", [False, True])
+def test_int4_values_under_every_scale(asym):
+    """Every nibble in every position of a word under each of the 65536 fp16 scale patterns (subnormals, infinities and NaN too;
+    with offsets, one of as many): the oracle's bits."""
+    hip = _hip()
+    rng = np.random.default_rng(77)
+    N, K = 65536, 32
+    q = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+    q[:, 0] = np.arange(N) & 255
+    s = np.arange(N, dtype=np.uint16).reshape(1, N)
+    z = rng.permutation(np.arange(N, dtype=np.uint16)).reshape(1, N) if asym else None
+    dq, ds = hip.DeviceArray.from_numpy(q), hip.DeviceArray.from_numpy(s)
+    dz = hip.DeviceArray.from_numpy(z) if asym else None
+    out = hip.DeviceArray((1, N, 32), np.float16)
+    hip.check(hip.lib().hxa_dequant(2, dq.ptr, ds.ptr, dz.ptr if dz else None, N, K, out.ptr, None), "dequant")
+    hip.sync()
+    ref = np.asarray(hxo.q4_dequant(q, s, z) if asym else hxo.q4_dequant(q, s)).view(np.float16).reshape(N, 32)
+    got = out.numpy()[0]
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got.view(np.uint16)[~nan], ref.view(np.uint16)[~nan])
