@@ -19,9 +19,10 @@ __global__ __launch_bounds__(256) void erf_t2_kernel(hxa_h *t) {
 // about rounds * (a * BM * BN * Kslice / 1e6 + b) + c microseconds. a, b, c >= 0 were fitted by least squares on the
 // relative error to every tile timed on 289 (M, N, K, slices) of 32 - 6656 rows on a 256-CU MI355X, weights k-tiled, each
 // launch repeated until the chip is at its power limit (where the block runner's chains keep it; a few launches after a
-// pause clock higher and rank the tiles differently). Over those shapes the picks come within 1.1% (fp16), 0.05% (int8)
-// and 0.1% (int4) of the fastest tile's summed time. a = 0 marks a tile that format does not use. nw is the wave count
-// under which hxa_gemm_tile takes the tile (tile_nw says what it runs on).
+// pause clock higher and rank the tiles differently). With weights that come cold from HBM, as a block's do, launches take 10 -
+// 40% longer than modelled, but the ranking holds: over 22 row counts x 15 shapes in one, two and four slices, cold weights,
+// the picks are 1.0% (fp16), 0.3% (int8) and 0.5% (int4) above the fastest tile (geometric mean). a = 0 marks a tile that
+// format does not use. nw is the wave count under which hxa_gemm_tile takes the tile (tile_nw says what it runs on).
 struct TileCost {
   int bm, bn, nw;
   float a[3], b[3], c[3];
@@ -52,29 +53,47 @@ int num_cu() {
 
 }  // namespace
 
-// Choose the tile of least modelled time (kTiles). HXA_EPI_RESADD_SPLIT2 keeps both K halves' accumulators in
-// registers and runs on the 4-wave 128x128 / 64x128 tiles only (ranked with the fp16 costs).
+// Choose the tile of least modelled time (kTiles). The model sees the rounds, not how much of them lies past the edges of M and
+// N; so of two tiles above 128x128 within 1% of each other the one that covers at least 8% less is taken (1152 rows x 8192
+// columns: 256x192 covers 1280 rows in 215 workgroups, 192x256 1152 in 192; int8, K 2048: 51.1 and 48.0 us, K 3072 x 9216 78.9
+// and 69.7. By any smaller difference there is nothing to gain: over 100 such pairs as many lose as win). HXA_EPI_RESADD_SPLIT2
+// keeps both K halves' accumulators in registers and runs on the 4-wave 128x128 / 64x128 tiles only (ranked with the fp16 costs).
 static void pick_tile(int M, int N, int K, int ksplit, int fmt, int epi, int hn_cols, int *bm, int *bn, int *nw) {
   const bool headnorm = hn_cols > 0;
   const bool split2 = epi == HXA_EPI_RESADD_SPLIT2;
   const int ncu = num_cu();
   const int f = split2 ? 0 : fmt;
-  double best = -1.0;
+  auto grid = [&](const TileCost &c) { return (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn); };
+  auto time = [&](const TileCost &c) {  // < 0: not for this GEMM
+    if (c.a[f] == 0.0f) return -1.0;
+    if (split2 && !(c.bn == 128 && (c.bm == 128 || c.bm == 64) && c.nw == 4)) return -1.0;  // register budget
+    if (epi == HXA_EPI_SITU && c.bn % 128 != 0) return -1.0;  // each wave needs whole (up, gate) block pairs
+    if (headnorm && (c.bn % 128 != 0 || (hn_cols % c.bn != 0 && hn_cols < N))) return -1.0;  // whole head-normed tiles
+    const long waves = (grid(c) * ksplit + ncu - 1) / ncu;
+    return (double)waves * (c.a[f] * 1e-6 * c.bm * c.bn * (double)(K / ksplit) + c.b[f]) + c.c[f];
+  };
+  auto covers = [&](const TileCost &c) { return (double)grid(c) * c.bm * c.bn; };
+  const TileCost *pick = nullptr;
+  double best = 0.0;
   for (const TileCost &c : kTiles) {
-    if (c.a[f] == 0.0f) continue;
-    if (split2 && !(c.bn == 128 && (c.bm == 128 || c.bm == 64) && c.nw == 4)) continue;  // register budget
-    if (epi == HXA_EPI_SITU && c.bn % 128 != 0) continue;  // each wave needs whole (up, gate) block pairs
-    if (headnorm && (c.bn % 128 != 0 || (hn_cols % c.bn != 0 && hn_cols < N))) continue;  // whole head-normed tiles
-    const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * ksplit;
-    const long waves = (tiles + ncu - 1) / ncu;
-    const double t = (double)waves * (c.a[f] * 1e-6 * c.bm * c.bn * (double)(K / ksplit) + c.b[f]) + c.c[f];
-    if (best < 0.0 || t < best - 1e-9) {
+    const double t = time(c);
+    if (t >= 0.0 && (pick == nullptr || t < best - 1e-9)) {
       best = t;
-      *bm = c.bm;
-      *bn = c.bn;
-      *nw = c.nw;
+      pick = &c;
     }
   }
+  if (pick == nullptr) return;
+  double least = 0.92 * covers(*pick);
+  for (const TileCost &c : kTiles) {
+    if (pick->bm * pick->bn <= 128 * 128 || c.bm * c.bn <= 128 * 128 || covers(c) >= least) continue;
+    const double t = time(c);
+    if (t < 0.0 || t > 1.01 * best) continue;
+    least = covers(c);
+    pick = &c;
+  }
+  *bm = pick->bm;
+  *bn = pick->bn;
+  *nw = pick->nw;
 }
 
 // the modelled time (us) of the tile pick_tile chooses for a plain-store GEMM with ksplit slices

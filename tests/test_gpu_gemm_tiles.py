@@ -232,3 +232,11 @@ def test_int4_values_under_every_scale(asym):
     nan = np.isnan(ref)
     assert np.array_equal(np.isnan(got), nan)
     assert np.array_equal(got.view(np.uint16)[~nan], ref.view(np.uint16)[~nan])
+
+
+@pytest.mark.parametrize("M,N,K,fmt,ks", [(1152, 8192, 2048, 1, 1), (1152, 2048, 8192, 1, 4), (1152, 9216, 3072, 2, 1)])
+def test_pick_covers_no_idle_rows_at_equal_cost(M, N, K, fmt, ks):
+    """256x192 and 192x256 tiles within 1% of each other in the model: the pick is the one whose tiles end with the rows."""
+    hip = _hip()
+    pk = hip.gemm_pick(M, N, K, fmt, ks, hip.EPI_PARTIAL if ks > 1 else 0)
+    assert (pk["bm"], pk["bn"]) == (192, 256)
