@@ -6,17 +6,18 @@
 // (export_all.py:31-32). Keys >= nvalid get probability 0.
 //
 // Work split: a workgroup of 2 x NWH waves (NWH = 4: 8 waves) owns 32 NWH = 128 queries of one head. Waves [0, NWH)
-// take the first half of the key tiles, the others the second half (two waves per SIMD, one of each half); the
-// halves are merged through LDS at the end. (96 queries on 6 waves would fill 256 CUs at 1536 queries x 16 heads,
-// but waves are dealt to the SIMDs round-robin, two SIMDs then run two waves, and the workgroup takes as long as
-// the 128-query one: 29.5 against 29.0 us on MI355X.) Each wave owns 32
+// take the first half of the key tiles, the others the second half; the halves are merged through LDS at the end. (96
+// queries on 6 waves would fill 256 CUs at 1536 queries x 16 heads, but waves are dealt to the SIMDs round-robin, two SIMDs then
+// run two waves, and the workgroup takes as long as the 128-query one: 29.5 against 29.0 us on MI355X.) Each wave owns 32
 // queries and keeps Q in registers. Schedules of the key loop: lock-step (one barrier per tile for both halves); for whole
-// tiles in an even number ping-pong (each tile split into a VALU phase, the softmax, and an MFMA
-// phase, PV with the next QK; the halves one phase apart, so the two waves of a SIMD alternate between the two
-// kinds of work: 5-6% faster at 1536 and 6656 keys on MI355X); and with 2 x 6 waves, 192 queries, three-phase (softmax, PV
-// and the next QK as phases of the three waves of a SIMD). What bounds them all is the softmax's VALU phase (about 1000
-// issue cycles per 32 x 64 scores, half of them v_exp_f32) and, beside it, LDS reads near 128 B / clk; queries_per_wg
-// chooses the workgroup that wastes least of the last round.
+// tiles in an even number ping-pong: each tile split into a VALU phase, the softmax, and an MFMA phase, PV with the next QK,
+// the halves one phase apart. With 128 queries waves w and w + 4 share a SIMD, one of each half, so it alternates between the
+// two kinds of work (5-6% faster at 1536 and 6656 keys on MI355X). With 64 queries (2 x 2 waves) every wave has a SIMD to
+// itself and nothing to alternate with; the phases then only keep the two halves' loads and LDS reads apart, which still beats
+// lock-step on the same grid (384 x 16 10.0 against 10.8 us, 1024 x 16 16.7 against 19.3). With 2 x 6 waves, 192 queries,
+// three-phase (softmax, PV and the next QK as phases of the three waves w, w + 4, w + 8 of a SIMD). What bounds them all is the
+// softmax's VALU phase (about 1000 issue cycles per 32 x 64 scores, half of them v_exp_f32); queries_per_wg chooses the
+// workgroup that wastes least of the last round.
 //
 // Per 64-key tile a wave computes S^T = K . Q^T (v_mfma_f32_32x32x16_f16), so a lane holds 16 scores of ONE query
 // and the row max needs a single exchange between the wave's two halves (v_permlane32_swap). K rows are stored in LDS with rows 4-7 and 8-11 of every 16 swapped,
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(2 * NWH * 64, 2) void attn_kernel(HxaAttn p, int nq
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // waves w and w + NWH share a SIMD (waves are dealt to the SIMDs round-robin): one wave of each key half
+  // waves are dealt to the SIMDs round-robin: with NWH = 4 the waves w and w + 4 of a SIMD belong to different key halves
   const int half = wave / NWH, wq = wave % NWH, g = lane >> 5, ql = lane & 31;
   // XCD-aware order: the query blocks of one head run on one XCD (its L2 keeps that head's K / V^T)
   const int ntot = nqb * p.H, bid = blockIdx.x;
@@ -316,9 +317,9 @@ __global__ __launch_bounds__(2 * NWH * 64, 2) void attn_kernel(HxaAttn p, int nq
   if constexpr (PP) {
     // Ping-pong form (both halves hold nh tiles, whole tiles): each tile is two phases, V(i) = the softmax of tile i
     // (VALU only: max, rescale, exponentials -> P(i)) and M(i) = its PV with the QK of tile i+1 (MFMA only), and
-    // half 1 runs one phase behind half 0. The waves of a SIMD belong to different halves (waves w and w + NWH), so
-    // in every phase one of them keeps the matrix core busy while the other computes exponentials. One workgroup
-    // barrier per phase (2 nh + 1 for either half).
+    // half 1 runs one phase behind half 0. With NWH = 4 the two waves of a SIMD belong to different halves, so
+    // in every phase one of them keeps the matrix core busy while the other computes exponentials (NWH = 2: one wave a
+    // SIMD). One workgroup barrier per phase (2 nh + 1 for either half).
     //  V(i) issues V(i+1) (its buffer held V(i-1), read in M(i-1)) and, from i = 1, K(i+2) (its buffer held K(i),
     //  read in M(i-1)); K(2) is issued in M(0), since half 0's QK of tile 0 has no barrier before V(0). Loads past
     //  the half's last tile reload that tile into the free buffer (M of the last tile skips its QK), so every V
@@ -427,8 +428,10 @@ __global__ __launch_bounds__(2 * NWH * 64, 2) void attn_kernel(HxaAttn p, int nq
     // runs V(i), P(i), Q(i) in the phases 3 i + ph, 3 i + 1 + ph, 3 i + 2 + ph; one workgroup barrier per phase.
     //  V^T(i) is read in the phases 3 i + 1 .. 3 i + 3, K(i + 1) in 3 i + 2 .. 3 i + 4, so phase g = 3 j + 1 issues
     //  V^T(j + 1) and g = 3 j + 2 issues K(j + 2), each into the buffer whose last reader finished a phase earlier. At the
-    //  end of phase 3 j (3 j + 1) a wave waits for its V^T(j) (K(j + 1)) loads: all but the youngest 4, which are
-    //  those of the K (V^T) tile after them (waves that load nothing have nothing to wait for).
+    //  end of phase 3 j (3 j + 1) a wave waits for its V^T(j) (K(j + 1)) loads: for all but the youngest 4, which are
+    //  those of the K (V^T) tile after them (waves that load nothing have nothing to wait for). A weight touch (PF) is one
+    //  load more among the younger ones, so those waits then take in one load of the next tile too (the touch a phase
+    //  later, behind the K loads: the same time, 2B fp16 blocks of 2112 - 3072 tokens within 0.5%).
     const int ph = wave >> 2, nph = 3 * nh + 2;
     half8_t pf[2][2];
     auto begin = [&](int g) {  // the loads of phase g

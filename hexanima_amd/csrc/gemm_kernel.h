@@ -8,7 +8,7 @@
 // Design (CDNA4, 64-wide waves):
 //  * 256 or 512 threads = 4 or 8 waves in a 2 x 2 or 2 x 4 grid over a BM x BN tile, v_mfma_f32_16x16x32_f16 with the
 //    weight fragment as the A operand (fp32 accumulate; each lane accumulates 4 consecutive output columns of a row).
-//  * K is consumed in stages of 64. A and W go from global memory straight into an LDS ring of 2 - 4 stages
+//  * K is consumed in stages of 64. A and W go from global memory straight into an LDS ring of 2 - 5 stages
 //    (global_load_lds_dwordx4, no VGPR staging); one s_barrier per stage, with explicit vmcnt waits so the prefetches
 //    stay in flight. 16-byte LDS chunks are XOR-swizzled per row so the fragment reads hit distinct banks.
 //  * int8 / int4 weights stay raw in LDS and are dequantised into the W fragments in registers with the fp16
@@ -218,8 +218,8 @@ struct GemmGeo {
   // Tiles below 128x128 have too few MFMAs per slice to cover an LDS read: they keep a whole stage of fragments ahead in
   // registers (gemm_body; 64x64 at K 8192: 32.6 -> 27.3 us)
   static constexpr bool DEEP = BM * BN < 128 * 128;
-  // ring stages: as many as fit in 160 KB, 4 at most; below 128x128 what lets two workgroups share a CU (64x128 with 6
-  // stages, one workgroup a CU: 9.6 -> 10.2 us at 512 x 2048 x 2048 in two K slices)
+  // ring stages: as many as fit in 160 KB, 4 at most; below 128x128 what lets two workgroups share a CU, 3, for 64x64 5 (64x128
+  // with 6 stages, one workgroup a CU: 9.6 -> 10.2 us at 512 x 2048 x 2048 in two K slices)
   static constexpr int NSMAX = BM * BN <= 64 * 64 ? 5 : BM * BN < 128 * 128 ? 3 : 4;
   static constexpr int NS = NSMAX * STAGE <= 160 * 1024 ? NSMAX : 3 * STAGE <= 160 * 1024 ? 3 : 2;
   static constexpr int lds(int ns) { return ns * STAGE > C_BYTES + PF_LDS ? ns * STAGE : C_BYTES + PF_LDS; }
@@ -712,8 +712,9 @@ HXA_DEV void xattn_tail(const GemmParams &p, const float4_t (&acc)[NI][MI], int 
 // loads) took, best tile to best tile, back to back: fp16 4096 x 2048 x 6144 115.6 -> 89.4 us, 1536 x 6144 x 2048 43.9 ->
 // 38.6, 256 x 2048 x 2048 15.5 -> 9.7; int8 1024 x 2048 x 8192 42.2 -> 36.7, 1536 x 10240 x 2560 81.1 -> 72.4.
 // k order: lane group h4 = lane / 16 takes the stage's k 16 h4 + 8 s .. + 7 in slice s, for A and W alike, so a lane's
-// int8 (int4) values of both slices are one 16-byte (8-byte) LDS read and belong to one quantisation group. Every
-// kernel uses this order, so a product's fp32 sums are the same whatever the tile.
+// int8 (int4) values of both slices are one 16-byte (8-byte) LDS read and belong to one quantisation group. Every tile
+// of this file uses this order, so its fp32 sums are the same whatever the tile; the skinny tiles (gemm_skinny.hip) use it within
+// each of the four K quarters that they add at the end.
 // An odd number of 32-k groups: stage 0 pairs group 0 with zeros, later stages start one group earlier.
 // SPLIT2: the first and second halves of K are rounded to fp16 separately and combined in the residual epilogue,
 // x += gate * (f16(first half) + f16(second half)) (blk.c:172-174 + kern.c:330-339 in one kernel): the first half's

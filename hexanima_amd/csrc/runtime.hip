@@ -499,9 +499,11 @@ struct WsLayout {
   long dq2_off, dq2_bytes;  // its second slot (text k / v weight)
 };
 // From this many rows on every int8 / int4 projection runs as one dequantisation pass into fp16 (WS_DQ) and the fp16
-// kernels; below, the GEMM dequantises under its MFMAs. Measured, int8, pass + fp16 against direct (us): 1024 x 2048 -> 2048
-// 20.4 / 18.5, 1568 x 3200 -> 3072 46.6 / 42.3, 4096 x 2048 -> 8192 128.6 / 125.7, 6656 x 3072 -> 3072 128.0 / 133.7, 6656 x
-// 12288 -> 3072 512 / 520; int4 at 6656 rows 1 - 9% in favour of the pass.
+// kernels; below, the GEMM dequantises under its MFMAs. Measured on whole blocks with cold weights, direct against pass (us a
+// block): 1024 - 2048 rows direct is 2 - 10% faster in every format and structure (2B int8 1536 rows 295 / 315, int4 288 /
+// 310; MOSS int8 + int4 2048 rows 710 / 746); 2304 - 4096 they are within 2% either way (2B int8 3072 rows 562 / 553, 4096 714 /
+// 715; 2.9B-class int4 3072 724 / 737); above, Anima blocks take 2 - 6% longer direct (2.9B int8 4608 rows 1192 / 1127, 6656
+// 1993 / 1926; int4 1946 / 1915), the wider MOSS blocks 0 - 3% less (6656 rows int8 + int4 2541 / 2570).
 constexpr long DQ_ROWS = 4096;
 // The fused cross attention takes fp16 weights only: from this many rows on its cross-q projection goes through the pass.
 constexpr long XDQ_ROWS = 1024;

@@ -214,8 +214,8 @@ def test_gemm_epilogues():
     W = f16(rng.standard_normal((N, K)) * 0.1)
     t = f16(hxo.gemm(A, W))
 
-    def t_gpu_for(epi):  # the GPU's own f16(acc) from a plain store on the tile the epilogue launch picks (kernels
-        pk = hip.gemm_pick(M, N, K, 0, 1, epi)  # differ in their k order, so f16(acc) may differ by an ulp)
+    def t_gpu_for(epi):  # the GPU's own f16(acc), which its fp32 sums may round an ulp from the oracle's, from a plain
+        pk = hip.gemm_pick(M, N, K, 0, 1, epi)  # store on the tile the epilogue launch picks
         return _run_gemm(hip, A, 0, W, None, N, K, tile=(pk["bm"], pk["bn"], pk["waves"]))
     say("gemm epi gelu tanh / erf")
     for epi, mode in ((1, 1), (2, 0)):
