@@ -12,8 +12,7 @@ __device__ __align__(16) hxa_h g_erf_t2[ERF_T2_N];
 __global__ __launch_bounds__(256) void erf_t2_kernel(hxa_h *t) {
   const int b = blockIdx.x * 256 + threadIdx.x;
   if (b >= ERF_T2_N) return;
-  const float a = (float)__builtin_bit_cast(hxa_h, (uint16_t)b);
-  t[b] = (hxa_h)(a * 0.5f * erfcf(a * 0.7071067811865476f));
+  t[b] = gelu_t2((float)__builtin_bit_cast(hxa_h, (uint16_t)b));
 }
 // Tile cost model, per weight format (fp16, int8, int4): a launch of `rounds` rounds of workgroups over the CUs takes
 // about rounds * (a * BM * BN * Kslice / 1e6 + b) + c microseconds. a, b, c >= 0 were fitted by least squares on the

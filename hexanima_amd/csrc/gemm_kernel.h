@@ -174,15 +174,14 @@ HXA_DEV float gelu_tanh_f(float t) {
   const float e = __builtin_amdgcn_exp2f(t * fmaf(K3, t * t, K1));
   return t * __builtin_amdgcn_rcpf(1.0f + e);  // v_rcp_f32 (1 ulp): far below the fp16 rounding
 }
-HXA_DEV float gelu_erf_f(float t) {
-  // kern.c:248-260: f16(max(t,0) - T2(|t|)), T2 = f16(|t| * 0.5 * erfc(|t|/sqrt 2))
-  const float a = fabsf(t);
-  const float t2 = (float)(hxa_h)(a * 0.5f * erfcf(a * 0.7071067811865476f));
-  return fmaxf(t, 0.0f) - t2;
+// T2(a) = f16(a * 0.5 * erfc(a / sqrt 2)) for a >= 0, 0 at infinity (where the product is inf * 0)
+HXA_DEV hxa_h gelu_t2(float a) { return a == INFINITY ? (hxa_h)0.0f : (hxa_h)(a * 0.5f * erfcf(a * 0.7071067811865476f)); }
+HXA_DEV float gelu_erf_f(float t) {  // kern.c:248-260: f16(max(t,0) - T2(|t|))
+  return fmaxf(t, 0.0f) - (float)gelu_t2(fabsf(t));
 }
-// T2(a) = f16(a * 0.5 * erfc(a / sqrt 2)) of gelu_erf_f for every non-negative fp16 bit pattern b (a = |t|; NaN and
-// inf patterns included): the GELU-erf epilogue looks its values up instead of evaluating erfcf per output. Filled
-// once per device by erf_t2_kernel with gelu_erf_f's own expression, so a lookup returns the same bits.
+// T2 of every non-negative fp16 bit pattern b (a = |t|; NaN and inf patterns included): the GELU-erf epilogue looks its values
+// up instead of evaluating erfcf per output. Filled once per device by erf_t2_kernel with gelu_t2, so a lookup returns the same
+// bits.
 constexpr int ERF_T2_N = 0x8000;
 // the part of the table a GELU-erf epilogue copies into LDS past its tile: 2^-11 <= |t| < 6 (bit patterns 0x1000 to
 // 0x4600), 27648 bytes = 27 wave-wide 16-byte copies, what 256x256 leaves of 160 KB; other |t| (rare) are looked up in the

@@ -153,8 +153,9 @@ def test_linear_takes_the_skinny_tile_for_few_output_tiles(fmt):
 
 @pytest.mark.parametrize("tile", [(256, 256, 9), (192, 256, 9), (128, 128, 4), (64, 64, 4)])
 def test_gelu_erf_over_every_fp16_value(tile):
-    """GELU-erf of every finite fp16 value and of infinities and NaN, which the LDS part of the lookup table (2^-11 <= |t| < 6)
-    and the global one share: within 2 ulps of the oracle (the fp16 rounding of T2 and of the result), the oracle's NaNs."""
+    """GELU-erf of every finite fp16 value, which the LDS part of the lookup table (2^-11 <= |t| < 6) and the global one share:
+    within 2 ulps of the oracle (the fp16 rounding of T2 and of the result); rows with a NaN or inf operand are NaN (inf * 0 in
+    the product). Infinities reach the epilogue in test_gelu_erf_of_overflowed_sums."""
     hip = _hip()
     say(f"gelu erf tile={tile}")
     M, N, K = 256, 256, 32
@@ -240,3 +241,23 @@ def test_pick_covers_no_idle_rows_at_equal_cost(M, N, K, fmt, ks):
     hip = _hip()
     pk = hip.gemm_pick(M, N, K, fmt, ks, hip.EPI_PARTIAL if ks > 1 else 0)
     assert (pk["bm"], pk["bn"]) == (192, 256)
+
+
+@pytest.mark.parametrize("tile", [(256, 256, 9), (128, 128, 4), (64, 64, 4)])
+def test_gelu_erf_of_overflowed_sums(tile):
+    """Products past the fp16 range reach the epilogue as infinities: GELU-erf of them is the oracle's inf and 0 (T2 is 0
+    there), beside finite values and NaN."""
+    hip = _hip()
+    M, N, K = 64, 64, 32
+    A = np.zeros((M, K), np.float16)
+    A[:, 0] = np.float16(60000.0)
+    A[1::4, 0] = np.float16(-60000.0)
+    A[2::4, 0] = np.float16(1.5)
+    A[3::4, 0] = np.float16(np.nan)
+    W = np.zeros((N, K), np.float16)
+    W[:, 0] = np.float16(2.0)
+    got = _run_gemm(hip, A, 0, W, None, N, K, epi=hip.EPI_GELU_ERF, tile=tile)
+    assert np.all(got[0::4] == np.inf) and np.all(got[1::4] == 0)
+    ref = hxo.gelu(np.full((1, 1), 3.0, np.float16), 0).view(np.float16)
+    assert ulp_diff(got[2::4], np.broadcast_to(ref, got[2::4].shape).copy()).max() <= 2
+    assert np.isnan(got[3::4]).all()
