@@ -43,6 +43,47 @@ def test_attention_forms(T, NKV, nvalid, H, batch):
         assert rel(g, exact) < 1e-3
 
 
+@pytest.mark.parametrize("T", [2304, 2176])
+def test_three_phase_attention_with_the_weight_touch(T):
+    """An fp16 Anima block (below 4096 rows its self attention touches the weights that follow) of as many tokens as take one
+    round of 192-query workgroups: after the attention stage, o equals, bit for bit, hxa_attention without the touch on the
+    block's own q, k and v, and a sample of its rows the oracle's exact softmax. The weights it touches stay as they are."""
+    from tests.test_gpu_block import make_anima_pack
+    hip = _hip()
+    say(f"three-phase attention with touch T={T}")
+    L = hip.lib()
+    rng = np.random.default_rng(T)
+    D, F, DC, C_ = 2048, 256, 128, 64
+    img, _, H = make_anima_pack(hip, rng, D, F, DC, 0)
+    x = rng.standard_normal((T, D)).astype(np.float32)
+    mod = (rng.standard_normal((9, D)) * 0.2).astype(np.float32)
+    ang = np.arange(T)[:, None] * 10000.0 ** (-np.arange(64) / 64.0)[None, :]
+    bufs = [hip.DeviceArray.from_numpy(a) for a in (img, f16(rng.standard_normal((C_, DC))), mod, np.cos(ang).astype(np.float32),
+                                                    np.sin(ang).astype(np.float32))]
+    d = hip.BlockDims(0, D, H, F, C_, DC, T, 1, T, 0, 0, 1)
+    ws, dx = hip.block_ws(d), hip.DeviceArray.from_numpy(x)
+    rec = hip.DeviceArray((1024, 4), np.uint64, zero=True)
+    hip.check(L.hxa_clock_record(1, rec.ptr, 1024), "clock_record")
+    try:
+        hip.check(L.hxa_block_run(C.byref(d), bufs[0].ptr, dx.ptr, bufs[1].ptr, bufs[2].ptr, bufs[3].ptr, bufs[4].ptr, ws.ptr, 4,
+                                  None, 0, None), "block_run")
+        hip.sync()
+    finally:
+        L.hxa_clock_record(1, None, 0)
+    assert np.count_nonzero(rec.numpy()[:, 0]) == -(-T // 192) * H  # the 192-query form
+    (q, ldq), (k, ldk), (vt, ldvt), (o, ldo) = (hip.ws_buffer(d, ws, w) for w in (hip.WS_Q, hip.WS_K, hip.WS_VT, hip.WS_O))
+    alone = hip.DeviceArray((T, D), np.float16)
+    hip.check(L.hxa_attention(q, ldq, k, ldk, vt, ldvt, alone.ptr, D, T, T, T, H, 1, 0, 0, 0, 0, None), "attention")
+    hip.sync()
+    got = hip.read_ws(d, ws, hip.WS_O, T, D)
+    assert np.array_equal(got.view(np.uint16), alone.numpy().view(np.uint16))
+    qh, kh, vh = (hip.read_ws(d, ws, w, r, c) for w, r, c in ((hip.WS_Q, T, D), (hip.WS_K, T, D), (hip.WS_VT, D, T)))
+    rows = np.unique(np.r_[np.arange(0, T, 97), T - 1])
+    exact = hxo.attention(np.ascontiguousarray(qh[rows]), kh, np.ascontiguousarray(vh.T), T, mode=1).view(np.float16)
+    assert rel(got[rows].astype(np.float64), exact.astype(np.float64)) < 1e-3
+    assert np.array_equal(bufs[0].numpy(), img)
+
+
 @pytest.mark.parametrize("lat_hw,wgs,alone", [((64, 32), 64, 128), ((64, 48), 96, 192)])
 def test_attention_that_hosts_the_modulation_keeps_128_queries(lat_hw, wgs, alone, monkeypatch):
     """2B-class DiT at 512 and 768 tokens, batch 1: the self-attention launch that streams the next block's modulation runs in

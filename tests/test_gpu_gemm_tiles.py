@@ -1,6 +1,8 @@
 """The GEMM kernels at the sizes where their pipelines can go wrong: odd numbers of 32-k groups, fewer stages than the ring
 holds, ragged rows and columns; the launches that must not depend on timing. Tolerance: assert_gemm_close (one fp16 ulp plus
 the fp32 accumulation-order error, tests/_helpers.py)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -66,8 +68,7 @@ def test_split_k_of_odd_slices(tile, fmt, asym):
 
 @pytest.mark.parametrize("fmt,M,N,K", [(1, 1536, 2560, 2560), (0, 512, 2048, 2048), (2, 300, 2048, 2048), (1, 64, 512, 8192)])
 def test_launches_repeat_bit_for_bit(fmt, M, N, K):
-    """40 launches on the same operands give the same bits, whatever runs beside them: a fragment read that the next stage's
-    loads could overtake shows as a difference."""
+    """40 launches on the same operands, one after another, at most a workgroup a CU, give the same bits."""
     hip = _hip()
     say(f"repeat fmt={fmt} {M}x{N}x{K}")
     L = hip.lib()
@@ -89,6 +90,65 @@ def test_launches_repeat_bit_for_bit(fmt, M, N, K):
                 b = o.numpy().view(np.uint16)
                 first = b if first is None else first
                 assert np.array_equal(b, first), (ks, rep)
+
+
+@pytest.mark.parametrize("tile,fmt,asym", [(t, f, a) for t in ((64, 64, 4), (64, 128, 4), (128, 64, 4)) for f, a in FORMATS
+                                           if not (f == 2 and t == (128, 64, 4))])  # (no such int4 kernel)
+def test_two_workgroups_a_cu_repeat_bit_for_bit(tile, fmt, asym):
+    """The tiles whose LDS ring lets two workgroups share a CU, on grids of two and more a CU: there the neighbour's loads put
+    lines into L1 that this workgroup's loads then find, and a stage lands soonest after its barrier. A fragment read that it
+    could overtake shows as a difference between launches."""
+    hip = _hip()
+    say(f"two workgroups a CU fmt={fmt} asym={asym} tile={tile}")
+    L = hip.lib()
+    rng = np.random.default_rng(720 + fmt + asym)
+    M, N, K = 2048, 2048, 2048
+    A = f16(rng.standard_normal((M, K)))
+    q, s, z, _ = _weights(rng, fmt, asym, N, K)
+    dA, dW = hip.DeviceArray.from_numpy(A), hip.DeviceArray.from_numpy(q)
+    dS = hip.DeviceArray.from_numpy(s) if s is not None else None
+    dZ = hip.DeviceArray.from_numpy(z) if z is not None else None
+    outs = [hip.DeviceArray((M, N), np.float16) for _ in range(8)]
+    first = None
+    for rep in range(3):
+        for o in outs:
+            hip.check(L.hxa_gemm_tile(dA.ptr, K, M, fmt, dW.ptr, dS.ptr if dS else None, dZ.ptr if dZ else None, N, K, 1, 0,
+                                      o.ptr, N, 0, None, 0, None, *tile, None), "gemm_tile")
+        hip.sync()
+        for o in outs:
+            b = o.numpy().view(np.uint16)
+            first = b if first is None else first
+            assert np.array_equal(b, first), rep
+
+
+@pytest.mark.parametrize("fmt,D,T,C_", [(1, 2560, 1536, 256), (0, 2560, 1792, 512), (2, 2560, 1536, 256)])
+def test_block_with_the_paired_launch_repeats_bit_for_bit(fmt, D, T, C_):
+    """The block whose cross q and text k / v run as one launch of more workgroups than CUs (2.9B class: 240 tiles and 80), 12
+    times on the same input: the same bits. There a stage's loads once overtook fragment reads of the GEMM loop."""
+    from tests.test_gpu_block import make_anima_pack
+    hip = _hip()
+    say(f"block repeat fmt={fmt} D={D} T={T}")
+    L = hip.lib()
+    rng = np.random.default_rng(740 + fmt)
+    F, DC = 1024, 1024
+    img, _, H = make_anima_pack(hip, rng, D, F, DC, fmt)
+    x = rng.standard_normal((T, D)).astype(np.float32)
+    mod = (rng.standard_normal((9, D)) * 0.2).astype(np.float32)
+    ang = np.arange(T)[:, None] * 10000.0 ** (-np.arange(64) / 64.0)[None, :]
+    bufs = [hip.DeviceArray.from_numpy(a) for a in (img, f16(rng.standard_normal((C_, DC))), mod, np.cos(ang).astype(np.float32),
+                                                    np.sin(ang).astype(np.float32))]
+    d = hip.BlockDims(0, D, H, F, C_, DC, T, 1, T, fmt, fmt, 1)
+    ws = hip.block_ws(d)
+    first = None
+    for rep in range(12):
+        dx = hip.DeviceArray.from_numpy(x)
+        hip.check(L.hxa_block_run(C.byref(d), bufs[0].ptr, dx.ptr, bufs[1].ptr, bufs[2].ptr, bufs[3].ptr, bufs[4].ptr, ws.ptr, 0,
+                                  None, 0, None), "block_run")
+        hip.sync()
+        b = dx.numpy().view(np.uint32)
+        assert np.isfinite(b.view(np.float32)).all()
+        first = b if first is None else first
+        assert np.array_equal(b, first), rep
 
 
 @pytest.mark.parametrize("fmt,asym", FORMATS)
