@@ -299,16 +299,20 @@ STAGES = ("LN-mod self", "qkv + head RMSNorm + RoPE (+ text k/v tiles)", "(RoPE:
           "(cross attention: fused)", "cross-o projection", "LN-mod MLP", "MLP up + GELU", "MLP down")
 FAMILIES = {  # family -> the stages whose launches it is
     "gemm_splitk": (4, 9, 12),
-    "gemm_pp_mlp_up": (11,),
-    "gemm_pp_qkv_headnorm": (1,),
+    "gemm_mlp_up": (11,),
+    "gemm_qkv_headnorm": (1,),
     "attention": (3,),
     "gemm_xattn_cross": (6,),
     "normrow": (0, 5, 10),
 }
 
 
-def _kname(pk):
-    return f"gemm_kernel {pk['bm']}x{pk['bn']} ({8 if pk['bm'] * pk['bn'] > 128 * 128 else 4} waves)"
+def _kname(pk, fmt=WFMT):
+    """the kernel of a picked tile with the waves it runs on (tile_nw in csrc/gemm_kernel.h; pick's 'waves' is only the tile's
+    name for hxa_gemm_tile)"""
+    area = pk["bm"] * pk["bn"]
+    waves = 8 if area > 128 * 128 or (pk["bn"] == 128 and fmt & 15 != 0) else 4
+    return f"gemm_kernel {pk['bm']}x{pk['bn']} ({waves} waves)"
 
 
 def family_launchers(L, hip, s):
@@ -394,17 +398,17 @@ def family_launchers(L, hip, s):
         "gemm_splitk": (splitk, 3, 2 * T * D * D * 2 + 2 * T * F * D,
                         f16 * (2 * (T * D + D * D + 2 * T * D) + (T * F + D * F + 2 * T * D)),
                         _kname(hip.gemm_pick(T, D, F, WFMT, 2, P)) + " split-K 2, fp16 partials"),
-        "gemm_pp_mlp_up": (mlp_up, 1, 2 * T * D * F, f16 * (T * D + F * D + T * F),
-                           _kname(hip.gemm_pick(T, F, D, WFMT, 1, hip.EPI_GELU_TANH)) + ", GELU epilogue"),
-        "gemm_pp_qkv_headnorm": (qkv, 1, 2 * T * D * 3 * D, f16 * (T * D + 3 * D * D + 3 * T * D),
-                                 _kname(hip.gemm_pick(T, 3 * D, D, WFMT, 1, 0, 2 * D)) + ", head RMSNorm + RoPE epilogue"
-                                 " (timed without the text k/v tiles the step's launch adds)"),
+        "gemm_mlp_up": (mlp_up, 1, 2 * T * D * F, f16 * (T * D + F * D + T * F),
+                        _kname(hip.gemm_pick(T, F, D, WFMT, 1, hip.EPI_GELU_TANH)) + ", GELU epilogue"),
+        "gemm_qkv_headnorm": (qkv, 1, 2 * T * D * 3 * D, f16 * (T * D + 3 * D * D + 3 * T * D),
+                              _kname(hip.gemm_pick(T, 3 * D, D, WFMT, 1, 0, 2 * D)) + ", head RMSNorm + RoPE epilogue"
+                              " (timed without the text k/v tiles the step's launch adds)"),
         "attention": (attention, 1, 4 * T * T * D, f16 * (4 * T * D), "attn_kernel (128-query workgroups)"),
         "gemm_xattn_cross": (xattn, 1, 2 * T * D * D + 4 * T * C_TXT * D, f16 * (T * D + D * D + 2 * C_TXT * D + T * D),
                              "gemm_xattn_kernel 128x128 (4 waves): cross q + head RMSNorm, attention over the text keys"),
     }
     for f, nm in ((0, "f16"), (1, "q8"), (2, "q4")):
-        picks = ", ".join(_kname(hip.gemm_pick(T, N, K, f, 1, 0)) for K, N in LIN_SHAPES)
+        picks = ", ".join(_kname(hip.gemm_pick(T, N, K, f, 1, 0), f) for K, N in LIN_SHAPES)
         fam["linears_" + nm] = (linears(f), len(LIN_SHAPES), lin_flops, lin_bytes[f],
                                 f"K x N {', '.join(f'{K}x{N}' for K, N in LIN_SHAPES)}: {picks}")
     # the MLP-down shape (K 8192, N 2048, 1536 rows) through hxa_linear: K slices into fp32 partials, then their sum
@@ -429,7 +433,7 @@ def family_launchers(L, hip, s):
                                    lws.ptr, lws.nbytes, s), "linear")
         fam["linear_split_" + nm] = (
             lin_run, 2, 2 * T * K * N, T * K * 2 + N * K * wb + (K // 32 * N * 2 if f else 0) + T * N * 2,
-            f"hxa_linear K x N {K}x{N}: {_kname(hip.gemm_pick(T, N, K, f, S, hip.EPI_PARTIAL_F32))} split-K {S} "
+            f"hxa_linear K x N {K}x{N}: {_kname(hip.gemm_pick(T, N, K, f, S, hip.EPI_PARTIAL_F32), f)} split-K {S} "
             f"(fp32 partials) + sum_partials_kernel")
     return fam, keep
 
@@ -731,7 +735,7 @@ def main():
     ap.add_argument("--kernel-probe", type=int, default=0, metavar="REPS",
                     help="only launch one kernel family REPS times plus a copy calibration (for rocprofv3 --pmc)")
     ap.add_argument("--probe-family", default="gemm_splitk",
-                    choices=["gemm_splitk", "gemm_pp_mlp_up", "gemm_pp_qkv_headnorm", "attention", "gemm_xattn_cross",
+                    choices=["gemm_splitk", "gemm_mlp_up", "gemm_qkv_headnorm", "attention", "gemm_xattn_cross",
                              "linears_f16", "linears_q8", "linears_q4", "linear_split_f16", "linear_split_q8",
                              "linear_split_q4"])
     ap.add_argument("--abi-chain", action="store_true", help="only time the 28-block mega_block chain (hxa_run)")
