@@ -695,7 +695,8 @@ bool ping_pong(int nvalid) { return nvalid % (2 * KT) == 0; }
 // Queries per workgroup of a launch past 256 keys.
 // 64 (4 waves, ping-pong) where their grid fits in one round: half the queries per SIMD, and twice the CUs (512 queries x 16
 // heads, 128 workgroups instead of 64: 12.8 -> 11.0 us; 1024 x 16 18.7 -> 16.5; as the second round begins it loses, 1536 x
-// 16 26.0 -> 38.6).
+// 16 26.0 -> 38.6). Masked keys or an odd number of tiles would take the lock-step loop, which gains little with 64 queries (384
+// x 16 11.8 -> 10.8) or loses (1024 x 16 18.7 -> 19.3), so they stay at 128.
 // 192 (12 waves, three-phase): a round takes about 1.45 times as long as one of 128 (12 key tiles a half: 39.4 us, 30.1),
 // so where they save more than a third of the rounds (1568 x 24: 216 workgroups in one round instead of 312 in two, 58.2 ->
 // 43.5 us; 3072 x 16: 256 instead of 384, 89.4 -> 81.6). With as many rounds, or 4 instead of 5, they are slower (6656 x 24:

@@ -145,7 +145,8 @@ int hxa_clock_record(int kind, void *rec, long nrec);
  * PARTIAL_F32: the same slices unrounded, ((float *)out)[z*out_zstride + m*ldo + n] (out 16-byte aligned, ldo % 4 == 0);
  * hxa_sum_partials adds them (hxa_linear's split-K form).
  * RESADD_SPLIT2 (ksplit 1, K % 128 == 0): x[m][n] += gate[n] (f16(first K/2) + f16(second K/2)), the split-K
- * down projection and its residual (blk.c:172-174, kern.c:330-339) in one launch. */
+ * down projection and its residual (blk.c:172-174, kern.c:330-339) in one launch.
+ * lda < 2^22; a row of w below 2^23 bytes, or k-tiled 32 k of the whole matrix below 4 GiB. */
 int hxa_gemm(const void *A, long lda, int M, int fmt, const void *w, const void *s, const void *z, int N, int K,
              int ksplit, int epi, void *out, long ldo, long out_zstride, float *x, long ldx, const float *gate,
              void *out_t, long ldo_t, int split_col, void *stream);
