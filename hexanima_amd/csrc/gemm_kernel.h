@@ -10,7 +10,11 @@
 //    weight fragment as the A operand (fp32 accumulate; each lane accumulates 4 consecutive output columns of a row).
 //  * K is consumed in stages of 64. A and W go from global memory straight into an LDS ring of 2 - 5 stages
 //    (global_load_lds_dwordx4, no VGPR staging); one s_barrier per stage, with explicit vmcnt waits so the prefetches
-//    stay in flight. 16-byte LDS chunks are XOR-swizzled per row so the fragment reads hit distinct banks.
+//    stay in flight. 16-byte LDS chunks are XOR-swizzled per row, which spreads one lane group's 16 rows over the banks; the
+//    passes of a ds_read_b128 mix two lane groups, whose rows still meet in pairs (SQ_LDS_BANK_CONFLICT is half of
+//    SQ_LDS_IDX_ACTIVE). A placement without these conflicts (bits 0 and 1 of the chunk exchanged before the XOR; counted: 0.04,
+//    LDS active 57 -> 29% of the MLP-down's cycles) leaves the times as they are, blocks fp16 0.0%, int8 -0.4%, int4 -1.5%,
+//    linears +0.1 / +0.1 / -0.6% (single ones +5%): LDS reads are not what the loops wait for.
 //  * int8 / int4 weights stay raw in LDS and are dequantised into the W fragments in registers with the fp16
 //    exponent-bias trick: a byte u placed under the exponent 0x64 is the fp16 value 1024+u, so (1024+u) - 1152 = q
 //    exactly, then one fp16 multiply by the group scale gives f16(q*s) -- the reference's exact dequantised value
@@ -751,7 +755,7 @@ HXA_DEV void gemm_body(const GemmParams &p, const int bid, const int z) {
   const int rot = XATTN ? (2 - nst) & 3 : 0;
 
   // ---- loader. 1 KB instruction t of a stage: 8 rows of A (t < NA) or 8 / 16 / 32 rows of fp16 / int8 / int4 W, 16
-  // bytes per lane, XOR-swizzled so that 16 rows' equal chunks (one LDS read) fall in distinct banks. The per-lane
+  // bytes per lane, XOR-swizzled so that 16 rows' equal chunks fall in distinct banks. The per-lane
   // offsets from the tile corner are fixed; a stage moves the wave-uniform bases. Rows past M / N clamp to the last.
   constexpr long ES = FMT == HXA_W_F16 ? 2 : 1;
   // group (0, 1) of the stage that this lane's chunk of instruction t belongs to
