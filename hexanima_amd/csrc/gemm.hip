@@ -18,24 +18,26 @@ __global__ __launch_bounds__(256) void erf_t2_kernel(hxa_h *t) {
 // about rounds * (a * BM * BN * Kslice / 1e6 + b) + c microseconds. a, b, c >= 0 were fitted by least squares on the
 // relative error to every tile timed on 289 (M, N, K, slices) of 32 - 6656 rows on a 256-CU MI355X, weights k-tiled, each
 // launch repeated until the chip is at its power limit (where the block runner's chains keep it; a few launches after a
-// pause clock higher and rank the tiles differently). With weights that come cold from HBM, as a block's do, launches take 10 -
-// 40% longer than modelled, but the ranking holds: over 22 row counts x 15 shapes in one, two and four slices, cold weights,
-// the picks are 1.0% (fp16), 0.3% (int8) and 0.5% (int4) above the fastest tile (geometric mean). a = 0 marks a tile that
-// format does not use. nw is the wave count under which hxa_gemm_tile takes the tile (tile_nw says what it runs on).
+// pause clock higher and rank the tiles differently); the int4 column (but 64x64) anew, the tiles near the fastest weighing
+// most, on 22 row counts x 15 shapes since its dequantisation takes 13 operations. With weights that come cold from HBM, as a
+// block's do, fp16 and int8 launches take 10 - 40% longer than modelled, but the ranking holds: over those 330 shapes in one,
+// two and four slices, cold weights, the picks are 1.0% (fp16), 0.3% (int8) and 0.4% (int4) above the fastest tile. a = 0
+// marks a tile that format does not use. nw is the wave count under which hxa_gemm_tile takes the tile (tile_nw says what it
+// runs on).
 struct TileCost {
   int bm, bn, nw;
   float a[3], b[3], c[3];
 };
 constexpr TileCost kTiles[] = {
-    {256, 256, 9, {0.2831f, 0.3081f, 0.3481f}, {7.81f, 8.13f, 8.15f}, {0.00f, 0.00f, 0.00f}},
-    {256, 192, 9, {0.3031f, 0.3574f, 0.3928f}, {6.67f, 7.38f, 7.46f}, {0.00f, 0.00f, 0.00f}},
-    {192, 256, 9, {0.3003f, 0.3604f, 0.3950f}, {6.89f, 7.32f, 7.21f}, {0.00f, 0.00f, 0.00f}},
-    {192, 192, 4, {0.3291f, 0.4331f, 0.4449f}, {6.27f, 6.77f, 6.58f}, {0.00f, 0.00f, 0.00f}},
-    {256, 128, 4, {0.3210f, 0.3878f, 0.4522f}, {5.91f, 6.09f, 6.30f}, {0.00f, 0.00f, 0.00f}},
-    {128, 256, 9, {0.3341f, 0.4520f, 0.5156f}, {6.10f, 6.37f, 5.95f}, {0.00f, 0.00f, 0.00f}},
-    {192, 128, 8, {0.3586f, 0.4163f, 0.4978f}, {5.60f, 5.81f, 5.61f}, {0.00f, 0.00f, 0.00f}},
-    {128, 128, 4, {0.4027f, 0.5403f, 0.7016f}, {4.98f, 4.81f, 4.05f}, {0.00f, 0.00f, 0.85f}},
-    {64, 128, 4, {0.5433f, 0.7834f, 0.8534f}, {1.64f, 0.78f, 0.31f}, {2.30f, 3.99f, 5.13f}},
+    {256, 256, 9, {0.2831f, 0.3081f, 0.3194f}, {7.81f, 8.13f, 12.77f}, {0.00f, 0.00f, 0.00f}},
+    {256, 192, 9, {0.3031f, 0.3574f, 0.3756f}, {6.67f, 7.38f, 10.18f}, {0.00f, 0.00f, 0.00f}},
+    {192, 256, 9, {0.3003f, 0.3604f, 0.3646f}, {6.89f, 7.32f, 10.46f}, {0.00f, 0.00f, 0.00f}},
+    {192, 192, 4, {0.3291f, 0.4331f, 0.4576f}, {6.27f, 6.77f, 8.13f}, {0.00f, 0.00f, 0.17f}},
+    {256, 128, 4, {0.3210f, 0.3878f, 0.4312f}, {5.91f, 6.09f, 8.46f}, {0.00f, 0.00f, 0.00f}},
+    {128, 256, 9, {0.3341f, 0.4520f, 0.4403f}, {6.10f, 6.37f, 8.09f}, {0.00f, 0.00f, 0.00f}},
+    {192, 128, 8, {0.3586f, 0.4163f, 0.4906f}, {5.60f, 5.81f, 6.87f}, {0.00f, 0.00f, 0.33f}},
+    {128, 128, 4, {0.4027f, 0.5403f, 0.6007f}, {4.98f, 4.81f, 5.00f}, {0.00f, 0.00f, 1.08f}},
+    {64, 128, 4, {0.5433f, 0.7834f, 0.8009f}, {1.64f, 0.78f, 0.59f}, {2.30f, 3.99f, 4.89f}},
     {128, 64, 4, {0.5638f, 0.6793f, 0.0000f}, {1.67f, 0.76f, 0.00f}, {2.00f, 4.33f, 0.00f}},
     {64, 64, 4, {0.7294f, 0.9569f, 0.9919f}, {1.14f, 0.62f, 0.00f}, {2.40f, 4.51f, 6.74f}},
 };
@@ -547,12 +549,12 @@ int hxa_sum_partials_launch(const float *p, int S, long zstride, long ldp, int M
 }
 
 // gemm_skinny_kernel's cost model, like kTiles: rounds * (a * K / 1000 + b) + c us, fitted to 16 - 1562 rows x 35 shapes
-// per format (cold weights, row counts up to 3 rounds)
+// per format (cold weights, row counts up to 3 rounds; int4 to 132 shapes since its dequantisation takes 13 operations)
 constexpr struct {
   int bm;
   double a[3], b[3], c[3];
-} kSkinny[] = {{64, {2.18, 2.00, 1.96}, {3.19, 3.48, 3.22}, {0.0, 0.0, 0.40}},
-               {32, {1.57, 1.59, 1.62}, {2.52, 2.39, 2.08}, {0.63, 1.05, 1.34}}};
+} kSkinny[] = {{64, {2.18, 2.00, 1.95}, {3.19, 3.48, 2.40}, {0.0, 0.0, 1.19}},
+               {32, {1.57, 1.59, 1.57}, {2.52, 2.39, 1.89}, {0.63, 1.05, 1.33}}};
 // the row count (64, 32) of the skinny tile whose modelled time is below t us, else 0
 static int skinny_rows(int M, int N, int K, int fmt, double t) {
   if (K % 64 != 0) return 0;
